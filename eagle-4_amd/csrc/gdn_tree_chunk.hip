@@ -1,6 +1,6 @@
 // GDN tree chunk form on the gfx950 matrix cores (kernels/gdn_tree_records.py:276-361, 496-579): the records
-// contract's verify without per-node rounding, for trees of at most 16 nodes, solved in closed form per (request,
-// value head) instead of walked node by node:
+// contract's verify without per-node rounding, solved in closed form per (request, value head) instead of walked node
+// by node (trees of at most 16 nodes first; gdn_chunk_wide_kernel takes up to 64):
 //
 //   R = strict-ancestor closure of the parent links,   G_t = product of exp(g) along t's root path,
 //   L = diag(beta) (R o G_t/G_j o K K^T),               D = (I + L)^-1 diag(beta) (V - diag(G) K S0^T),
@@ -49,8 +49,7 @@ E4_DEV f32x4_t mma_bf16(uint4 a, uint4 b, f32x4_t c) {
 // X Y for 16 x 16 fp32 matrices in the accumulator layout, X passed transposed: block kb of the 16x16x4 MFMA
 // contracts over k = 4 g + kb, for which a lane's A operand X[c][4 g + kb] is element kb of its X^T and its B operand
 // Y[4 g + kb][c] element kb of its Y.
-E4_DEV f32x4_t mm(f32x4_t xt, f32x4_t y) {
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+E4_DEV f32x4_t mm(f32x4_t xt, f32x4_t y, f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f}) {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[kb], y[kb], acc, 0, 0, 0);
   return acc;
@@ -414,19 +413,401 @@ int launch_k(const eagle4_records_args& a, hipStream_t s) {
   return launch_pool<K, 1>(a, s);
 }
 
+// ---- trees of 17 to 64 nodes ---------------------------------------------------------------------------------------
+// The same closed form, blocked by tiles of 16 nodes: with every parent in front of its children L is block lower
+// triangular, so the tiles are solved in order,
+//   D_I = (I + L_II)^-1 (rhs_I - sum_{J<I} L_IJ D_J),   O_I = diag(G) Q_I S0^T + sum_{J<=I} W_IJ D_J,
+// each 16 x 16 block on the MFMA as above, the blocks of tile I built when it is solved (they are used at once by the
+// wave's NTL column tiles, nothing is kept but D). One wave per (request, value head, 16 NTL columns). Rows given in
+// another order are first ranked by depth. Bound by the fp32 MFMA (about 350 of 32 cycles per wave at 4 tiles and two
+// column tiles) and, with few requests, by their dependence; the walk that it replaces steps through the nodes one by
+// one, each a chain of two lane sums. K = V = 128, fp32 pool, one call among others: 1 request of 24 nodes, 16 heads
+// 33.4 -> 9.4 us; 8 of 40 nodes, 48 heads 318 -> 31 us; 32 of 64 nodes, 48 heads 2108 -> 157 us.
+//   - Decay ratios are exp2 of differences of root-path sums of log2 decays; the sums are fp64, so what two nodes share
+//     cancels exactly and the ratio's error is that of the path between them, whatever the root path's length.
+//   - A value that is not finite stays on its node and the node's descendants, as in a walk: products with zeros would
+//     spread it over the tile, so it is taken out of the right-hand sides (and a node with such a key or gate out of
+//     the products), remembered per column, and put back as NaN where the outputs of that path are stored.
+template <int K, int NTL, int NTILE, typename Tpool>
+__global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records_args a, int slices, int per_xcd,
+                                                             int total) {
+  constexpr int KB = K / 32;
+  constexpr int NN = 16 * NTILE;
+  constexpr int ROUNDS = NN <= 32 ? 5 : 6;  // pointer jumping: depth < 2^ROUNDS
+  using PT = PoolTerms<Tpool>;
+  __shared__ float4 s_nd[64];     // per node: ks, qs, beta, G
+  __shared__ double s_lg[64];     // per node: log2 G
+  __shared__ uint64_t s_anc[64];  // per node: strict ancestors
+  __shared__ float2 s_nrm[64];    // per node: |k|^2, |q|^2
+  __shared__ int s_id[64];        // position -> row of the request
+
+  const int w = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
+  if (w >= total) return;
+  const int slice = w % slices, pair = w / slices;
+  const int hv = pair % a.HV, n = pair / a.HV;
+  const int ih = hv / (a.HV / a.H);
+  const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+
+  const int qs0 = entry(a.query_start_loc, n), qs1 = entry(a.query_start_loc, n + 1);
+  const int rec_row = uni(entry(a.record_indices, n));
+  const int idx = uni(entry(a.state_indices, n));
+  const Word A_w = word_of(a.A_log, hv, a.A_log_dtype);
+  const Word dt_w = word_of(a.dt_bias, hv, a.dt_bias_dtype);
+  const int64_t bos = uni(qs0);
+  int T = uni(qs1) - uni(qs0);
+  T = T < a.width ? T : a.width;  // a tree has at most width (<= 16 NTILE) rows
+  if (T <= 0) return;
+
+  // ---- every load before the first wait; rows past the tree read its last row (masked below) ------------------------
+  const int par_raw = entry(a.parent, n, lane < T ? lane : T - 1);
+  uint4 qr[NTILE][KB], kr[NTILE][KB];
+  Run16<NTL> vr[NTILE][4];
+  Word ga, gb;
+  const int v0 = slice * 16 * NTL;
+  auto load_rows = [&](auto&& row_of) {  // row_of(position): the request's row there
+    const int64_t tl = bos + row_of(lane < T ? lane : T - 1);
+    ga = word_of(a.a, tl * a.stride_a + hv, a.gate_dtype);
+    gb = word_of(a.b, tl * a.stride_b + hv, a.gate_dtype);
+#pragma unroll
+    for (int I = 0; I < NTILE; ++I) {
+      const int p = 16 * I + c;
+      const int64_t tok = bos + row_of(p < T ? p : T - 1);
+      const uint16_t* qp = static_cast<const uint16_t*>(a.q) + tok * a.stride_q + ih * K + 8 * g;
+      const uint16_t* kp = static_cast<const uint16_t*>(a.k) + tok * a.stride_k + ih * K + 8 * g;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        qr[I][kb] = *reinterpret_cast<const uint4*>(qp + 32 * kb);
+        kr[I][kb] = *reinterpret_cast<const uint4*>(kp + 32 * kb);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * I + 4 * g + r;
+        const int64_t ti = bos + row_of(i < T ? i : T - 1);
+        vr[I][r].load(static_cast<const uint16_t*>(a.v) + ti * a.stride_v + static_cast<int64_t>(hv) * a.V + v0 + NTL * c);
+      }
+    }
+  };
+  load_rows([](int p) { return p; });
+  using PS = typename Tpool::storage;
+  constexpr int kSliceBytes = 16 * NTL * K * static_cast<int>(sizeof(PS));
+  const char* slot = static_cast<const char*>(a.state) +
+                     ((idx >= 0 ? static_cast<int64_t>(idx) * a.stride_state : 0) +
+                      (static_cast<int64_t>(hv) * a.V + v0) * K) * static_cast<int64_t>(sizeof(PS));
+  const __amdgpu_buffer_rsrc_t srsrc =  // empty for a negative slot: zeros
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(slot), 0, idx >= 0 ? kSliceBytes : 0, 0x00020000);
+  uint4 sraw[NTL][KB][PT::WORDS];
+#pragma unroll
+  for (int u = 0; u < NTL; ++u)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int q = 0; q < PT::WORDS; ++q) {
+        const int off = ((NTL * c + u) * K + 32 * kb + 8 * g) * static_cast<int>(sizeof(PS)) + 16 * q;
+        sraw[u][kb][q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(srsrc, off, 0, 0));
+      }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the order of the nodes: parents first -------------------------------------------------------------------------
+  // lane p is the node at position p; a parent outside the tree (or the node itself) makes the node a root
+  int par = lane > 0 && lane < T && par_raw >= 0 && par_raw < T && par_raw != lane ? par_raw : -1;
+  const bool reordered = __ballot(par > lane) != 0;
+  s_id[lane] = lane;
+  if (reordered) {  // rank the rows by (depth, row)
+    int depth = 0;
+    for (int it = 0, x = par; it < T; ++it) {  // one step up for every lane; all lanes take part in the shuffle
+      const int up = __shfl(par, x >= 0 ? x : 0);
+      if (x >= 0) {
+        ++depth;
+        x = up;
+      }
+    }
+    const int key = lane < T ? depth * 64 + lane : 64 * 128 + lane;
+    int rank = 0;
+    for (int j = 0; j < 64; ++j) rank += readlane(key, j) < key ? 1 : 0;
+    s_id[rank] = lane;
+    __syncthreads();
+    const int parent_rank = __shfl(rank, par >= 0 ? par : 0);
+    const int by_row = par >= 0 ? parent_rank : -1;
+    par = __shfl(by_row, s_id[lane]);
+    load_rows([&](int p) { return s_id[p]; });
+  }
+
+  // ---- per node (lane p): gates, ancestors, root-path log decay; squared norms from the tiles' diagonals --------------
+  const float A = -expf(widen_word(A_w, a.A_log_dtype));
+  const float dt_bias = widen_word(dt_w, a.dt_bias_dtype);
+#pragma unroll
+  for (int I = 0; I < NTILE; ++I) {
+    f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, QQ = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      KK = mma_bf16(kr[I][kb], kr[I][kb], KK);
+      QQ = mma_bf16(qr[I][kb], qr[I][kb], QQ);
+    }
+    const int rc = c & 3;
+    const float kk = rc == 0 ? KK[0] : rc == 1 ? KK[1] : rc == 2 ? KK[2] : KK[3];
+    const float qq = rc == 0 ? QQ[0] : rc == 1 ? QQ[1] : rc == 2 ? QQ[2] : QQ[3];
+    if (g == (c >> 2)) s_nrm[16 * I + c] = make_float2(kk, qq);
+  }
+  const float2 gt = gate_of(a.gate_dtype == EAGLE4_F32 ? ga.w : (ga.w >> ga.sh) & 0xffffu,
+                            a.gate_dtype == EAGLE4_F32 ? gb.w : (gb.w >> gb.sh) & 0xffffu, a.gate_dtype, 1.0f, 20.0f,
+                            A, dt_bias);
+  const float x_dt = widen_word(ga, a.gate_dtype) + dt_bias;
+  const float gl = A * (x_dt <= 20.0f ? logf(1.0f + expf(x_dt)) : x_dt);  // gate_of's log decay
+  uint64_t anc = par >= 0 ? 1ull << par : 0ull;
+  int jmp = par;
+  double lsum = lane < T ? fmax(static_cast<double>(gl) * 1.4426950408889634, -1048576.0) : 0.0;
+#pragma unroll
+  for (int it = 0; it < ROUNDS; ++it) {
+    const int src = jmp >= 0 ? jmp : lane;
+    const uint32_t lo = static_cast<uint32_t>(__shfl(static_cast<int>(anc & 0xffffffffu), src));
+    const uint32_t hi = NN > 32 ? static_cast<uint32_t>(__shfl(static_cast<int>(anc >> 32), src)) : 0u;
+    const int jmp_j = __shfl(jmp, src);
+    const double l_j = __shfl(lsum, src);
+    if (jmp >= 0) {
+      anc |= (static_cast<uint64_t>(hi) << 32) | lo;
+      lsum += l_j;
+      jmp = jmp_j;
+    }
+  }
+  __syncthreads();
+  const float2 nrm = s_nrm[lane < NN ? lane : 0];
+  const float ks_l = 1.0f / sqrtf(nrm.x + 1e-6f);
+  const bool finite = fabsf(nrm.x) <= 3.4e38f && fabsf(gt.x) <= 3.4e38f && fabsf(gt.y) <= 3.4e38f;
+  const uint64_t bad = __ballot(lane < T && !finite);  // nodes whose key or gate is not finite
+  const bool use = lane < T && finite;
+  s_nd[lane] = make_float4(use ? ks_l : 0.f, a.scale / sqrtf(nrm.y + 1e-6f), use ? gt.y : 0.f,
+                           __builtin_amdgcn_exp2f(static_cast<float>(lsum)));
+  s_lg[lane] = lsum;
+  s_anc[lane] = anc;
+  __syncthreads();
+  // the records' keys and decays (once per node and value head) leave ahead of the matrix work
+  float* rec = a.records + static_cast<int64_t>(rec_row) * a.stride_records_row;
+  if (slice == 0 && rec_row >= 0) {
+#pragma unroll
+    for (int I = 0; I < NTILE; ++I) {
+      const int p = 16 * I + c;
+      if (p < T) {
+        float* d0 = rec + (static_cast<int64_t>(s_id[p]) * a.HV + hv) * a.rec + a.V;
+        const float ks = 1.0f / sqrtf(s_nrm[p].x + 1e-6f);
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const uint4 x = kr[I][kb];
+          float4* d = reinterpret_cast<float4*>(d0 + 32 * kb + 8 * g);
+          d[0] = make_float4(lo_bf16(x.x) * ks, hi_bf16(x.x) * ks, lo_bf16(x.y) * ks, hi_bf16(x.y) * ks);
+          d[1] = make_float4(lo_bf16(x.z) * ks, hi_bf16(x.z) * ks, lo_bf16(x.w) * ks, hi_bf16(x.w) * ks);
+        }
+      }
+    }
+    if (lane < T) rec[(static_cast<int64_t>(s_id[lane]) * a.HV + hv) * a.rec + a.V + K] = gt.x;
+  }
+  if (bad != 0) {
+#pragma unroll
+    for (int I = 0; I < NTILE; ++I)
+      if ((bad >> (16 * I + c)) & 1) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) kr[I][kb] = make_uint4(0u, 0u, 0u, 0u);
+      }
+  }
+
+  // ---- K S0^T and Q S0^T of every tile -------------------------------------------------------------------------------
+  f32x4_t KS[NTILE][NTL], QS[NTILE][NTL];
+#pragma unroll
+  for (int I = 0; I < NTILE; ++I)
+#pragma unroll
+    for (int u = 0; u < NTL; ++u) {
+      KS[I][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      QS[I][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+  for (int u = 0; u < NTL; ++u)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      uint4 st[PT::N];
+      PT::split(sraw[u][kb], st);
+#pragma unroll
+      for (int s = 0; s < PT::N; ++s)
+#pragma unroll
+        for (int I = 0; I < NTILE; ++I) {
+          KS[I][u] = mma_bf16(kr[I][kb], st[s], KS[I][u]);
+          QS[I][u] = mma_bf16(qr[I][kb], st[s], QS[I][u]);
+        }
+    }
+
+  // ---- the tiles in order ---------------------------------------------------------------------------------------------
+  f32x4_t D[NTILE][NTL];
+  uint64_t lost[NTL];  // column v0 + NTL c + u: the nodes whose right-hand side is not finite
+#pragma unroll
+  for (int u = 0; u < NTL; ++u) lost[u] = 0;
+  bool any_lost = bad != 0;
+#pragma unroll
+  for (int I = 0; I < NTILE; ++I) {
+    if (16 * I >= T) break;
+    const float4 ci = s_nd[16 * I + c];  // the node of this lane's column
+    const double lg_c = s_lg[16 * I + c];
+    const uint64_t anc_c = s_anc[16 * I + c];
+    f32x4_t sub[NTL], out[NTL];
+#pragma unroll
+    for (int u = 0; u < NTL; ++u) {
+      sub[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      out[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int J = 0; J < I; ++J) {
+      f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, KQ = {0.f, 0.f, 0.f, 0.f}, LT, WT;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        KK = mma_bf16(kr[J][kb], kr[I][kb], KK);
+        KQ = mma_bf16(kr[J][kb], qr[I][kb], KQ);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = 16 * J + 4 * g + r;
+        const float ks_j = s_nd[j].x;
+        const float ratio = __builtin_amdgcn_exp2f(static_cast<float>(lg_c - s_lg[j]));
+        const bool above = (anc_c >> j) & 1;
+        LT[r] = above ? ci.z * ratio * (ks_j * ci.x * KK[r]) : 0.f;  // L^T: L[c][j]
+        WT[r] = above ? ratio * (ci.y * ks_j * KQ[r]) : 0.f;         // W^T
+      }
+#pragma unroll
+      for (int u = 0; u < NTL; ++u) {
+        sub[u] = mm(LT, D[J][u], sub[u]);
+        out[u] = mm(WT, D[J][u], out[u]);
+      }
+    }
+    f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, KQ = {0.f, 0.f, 0.f, 0.f}, L, LT, WT, E;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      KK = mma_bf16(kr[I][kb], kr[I][kb], KK);
+      KQ = mma_bf16(kr[I][kb], qr[I][kb], KQ);
+    }
+    float4 nd[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 4 * g + r, ni = 16 * I + i;
+      nd[r] = s_nd[ni];
+      const double lg_i = s_lg[ni];
+      const bool c_above_i = (s_anc[ni] >> (16 * I + c)) & 1, i_above_c = (anc_c >> ni) & 1;
+      const float kk_n = nd[r].x * ci.x * KK[r];
+      L[r] = c_above_i ? nd[r].z * __builtin_amdgcn_exp2f(static_cast<float>(lg_i - lg_c)) * kk_n : 0.f;
+      const float ratio = i_above_c || i == c ? __builtin_amdgcn_exp2f(static_cast<float>(lg_c - lg_i)) : 0.f;
+      LT[r] = i_above_c ? ci.z * ratio * kk_n : 0.f;
+      WT[r] = i_above_c || i == c ? ratio * (ci.y * nd[r].x * KQ[r]) : 0.f;
+      E[r] = i == c ? 1.f : 0.f;
+    }
+    const f32x4_t P2 = mm(LT, L), P2T = mm(L, LT);
+    const f32x4_t P4 = mm(P2T, P2), P4T = mm(P2, P2T);
+    const f32x4_t P8 = mm(P4T, P4);
+    f32x4_t TinvT = mm(E + P2, E - LT);
+    TinvT = mm(E + P4, TinvT);
+    TinvT = mm(E + P8, TinvT);
+#pragma unroll
+    for (int u = 0; u < NTL; ++u) {
+      f32x4_t rhs;
+      bool off = false;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        rhs[r] = 16 * I + 4 * g + r < T
+                     ? nd[r].z * (vr[I][r].at(u) - nd[r].w * (nd[r].x * KS[I][u][r])) - sub[u][r] : 0.f;
+        off |= !(fabsf(rhs[r]) <= 3.4e38f);
+      }
+      if (__ballot(off) != 0) {  // take what is not finite out of the products, remember where it was
+        uint32_t m = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!(fabsf(rhs[r]) <= 3.4e38f)) {
+            m |= 1u << (4 * g + r);
+            rhs[r] = 0.f;
+          }
+        m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16));
+        m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32));
+        lost[u] |= static_cast<uint64_t>(m) << (16 * I);
+        any_lost = true;
+      }
+      D[I][u] = mm(TinvT, rhs);
+      out[u] = mm(WT, D[I][u], out[u]);
+    }
+    // ---- the tile's outputs and deltas ----
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p = 16 * I + 4 * g + r;
+      if (p >= T) continue;
+      float o[NTL], d[NTL];
+#pragma unroll
+      for (int u = 0; u < NTL; ++u) {
+        o[u] = nd[r].w * (nd[r].y * QS[I][u][r]) + out[u][r];
+        d[u] = D[I][u][r];
+      }
+      if (any_lost) {
+        const uint64_t path = s_anc[p] | (1ull << p);
+#pragma unroll
+        for (int u = 0; u < NTL; ++u)
+          if ((path & (lost[u] | bad)) != 0) o[u] = d[u] = __builtin_nanf("");
+      }
+      const int row = s_id[p];
+      const int64_t col = static_cast<int64_t>(hv) * a.V + v0 + NTL * c;
+      store_run_out<NTL>(a.out, (bos + row) * a.stride_o + col, a.out_dtype, o);
+      if (rec_row >= 0) store_run_f32<NTL>(rec + (static_cast<int64_t>(row) * a.HV + hv) * a.rec + v0 + NTL * c, d);
+    }
+  }
+}
+
+template <int K, int NTL, int NTILE>
+int launch_wide_pool(const eagle4_records_args& a, hipStream_t s) {
+  const int slices = a.V / (16 * NTL);
+  const int64_t total = static_cast<int64_t>(a.N) * a.HV * slices;
+  if (total > (int64_t(1) << 30)) return EAGLE4_NOT_COVERED;
+  const int per_xcd = static_cast<int>((total + 7) / 8);
+  const int t = static_cast<int>(total);
+  if (a.state_dtype == EAGLE4_BF16)
+    gdn_chunk_wide_kernel<K, NTL, NTILE, e4::Bf16><<<8 * per_xcd, 64, 0, s>>>(a, slices, per_xcd, t);
+  else if (a.state_dtype == EAGLE4_F16)
+    gdn_chunk_wide_kernel<K, NTL, NTILE, e4::F16><<<8 * per_xcd, 64, 0, s>>>(a, slices, per_xcd, t);
+  else if (a.state_dtype == EAGLE4_F32)
+    gdn_chunk_wide_kernel<K, NTL, NTILE, e4::F32><<<8 * per_xcd, 64, 0, s>>>(a, slices, per_xcd, t);
+  else
+    return EAGLE4_NOT_COVERED;
+  return E4_LAUNCH_STATUS();
+}
+
+// Two column tiles per wave halve the work on the node blocks that the waves of a head repeat, one gives twice the
+// waves: from 512 waves of two on, two are faster (32 requests of 64 nodes, 48 heads 157 against 205 us; 8 of 24 nodes,
+// 16 heads: 512 waves, 12.9 against 12.2, of 64 nodes 24.8 against 24.7; 2 of 64 nodes, 48 heads: 384 waves, 23.7
+// against 21.3).
+template <int K, int NTILE>
+int launch_wide(const eagle4_records_args& a, hipStream_t s) {
+  const int64_t pairs = static_cast<int64_t>(a.N) * a.HV;
+  if (a.V % 32 == 0 && pairs * (a.V / 32) >= 512) return launch_wide_pool<K, 2, NTILE>(a, s);
+  return launch_wide_pool<K, 1, NTILE>(a, s);
+}
+
+template <int K>
+int launch_wide_k(const eagle4_records_args& a, hipStream_t s) {
+  if (a.width <= 32) return launch_wide<K, 2>(a, s);
+  if (a.width <= 48) return launch_wide<K, 3>(a, s);
+  return launch_wide<K, 4>(a, s);
+}
+
 }  // namespace
 
 namespace e4chunk {
 
-// The chunk form on the matrix cores when it covers the call: no path table, trees of <= 16 nodes, bf16 inputs, a
-// key dim that is a multiple of 32 (<= 256), value dim a multiple of 16, 16-byte aligned rows. Returns
-// EAGLE4_NOT_COVERED (nothing launched) otherwise.
+// The chunk form on the matrix cores when it covers the call: no path table, bf16 inputs, a key dim of 32 .. 256 for
+// trees of <= 16 nodes and of 32 .. 128 up to 64 nodes (four tiles of 256-wide rows would not fit the registers), value
+// dim a multiple of 16, 16-byte aligned rows. Returns EAGLE4_NOT_COVERED (nothing launched) otherwise.
 int launch(const eagle4_records_args& a, hipStream_t s) {
   const auto al = [](const void* p, int64_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
-  if (a.path_replay || a.width > NP || a.in_dtype != EAGLE4_BF16 || a.V % 16 || a.stride_q % 8 || a.stride_k % 8 ||
+  if (a.path_replay || a.width > 64 || a.in_dtype != EAGLE4_BF16 || a.V % 16 || a.stride_q % 8 || a.stride_k % 8 ||
       a.stride_v % 4 || a.stride_o % 4 || a.rec % 4 || a.stride_records_row % 4 || !al(a.q, 16) || !al(a.k, 16) ||
       !al(a.v, 8) || !al(a.out, 16) || !al(a.records, 16) || !al(a.state, 16) || a.stride_state % 8)
     return EAGLE4_NOT_COVERED;
+  if (a.width > NP) {
+    switch (a.K) {
+      case 32: return launch_wide_k<32>(a, s);
+      case 64: return launch_wide_k<64>(a, s);
+      case 128: return launch_wide_k<128>(a, s);
+      default: return EAGLE4_NOT_COVERED;
+    }
+  }
   switch (a.K) {
     case 32: return launch_k<32>(a, s);
     case 64: return launch_k<64>(a, s);

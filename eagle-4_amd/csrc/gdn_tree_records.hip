@@ -20,7 +20,7 @@
 #include "gdn_walk.h"
 
 namespace e4chunk {
-// gdn_tree_chunk.hip: the chunk form on the matrix cores (trees of <= 16 nodes, bf16 inputs)
+// gdn_tree_chunk.hip: the chunk form on the matrix cores (bf16 inputs; K <= 128 above 16 nodes)
 int launch(const eagle4_records_args& a, hipStream_t s) __attribute__((visibility("hidden")));
 }
 namespace e4replay {

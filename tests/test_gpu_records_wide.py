@@ -1,0 +1,60 @@
+"""The chunk form of trees of 17 to 64 nodes on the matrix cores: tile edges, rows in any order, every pool dtype,
+against the oracle's closed form (fp32 records within 1e-4, as the narrower trees'), and values that are not finite,
+which reach the node they are given to and its descendants only."""
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce
+from test_gpu_records import _call, _chunk_case, _inputs, _relabelled_tree, _to
+from workloads import seeded_tree
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width,dims,pool_dtype", [
+    (17, (2, 4, 128, 128), torch.float32), (31, (1, 3, 64, 48), torch.bfloat16), (32, (2, 2, 128, 32), torch.float16),
+    (33, (1, 2, 32, 16), torch.float32), (48, (2, 4, 128, 64), torch.bfloat16), (49, (1, 2, 64, 32), torch.float32),
+    (64, (2, 4, 128, 128), torch.float32), (64, (1, 2, 128, 32), torch.float16)])
+def test_wide_trees_match_the_closed_form(dev, width, dims, pool_dtype):
+    announce(f"records chunk form width {width} dims={dims} pool={pool_dtype}")
+    rng = np.random.default_rng(width)
+    trees = [seeded_tree(rng, width), _relabelled_tree(rng, width), list(range(-1, width - 1)), [-1], [],
+             seeded_tree(rng, 16), _relabelled_tree(rng, width - 1), seeded_tree(rng, width - 2)]
+
+    def edit(inp):
+        inp["state_indices"][6] = -1  # no pool slot: zeros
+        inp["record_indices"][7] = -1  # outputs only
+
+    _chunk_case(dev, trees, dims, pool_dtype, width, edit)
+
+
+@pytest.mark.parametrize("what", ["v", "k", "a"])
+def test_values_that_are_not_finite_stay_on_their_path(dev, what):
+    """One node's value, key or gate not finite: the node and its descendants get outputs that are not finite in the
+    columns concerned, every other output keeps its bits."""
+    from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
+
+    announce(f"records chunk form, {what} not finite")
+    tree = [-1, 0, 1, 2, 0, 4, 5] + list(range(6, 30)) + [0, 31, 32]  # node 3's chain ends; 4 .. 30 one chain; 31 .. 33
+    inp, width = _inputs([tree], 1, 2, 128, 32, torch.float32, seed=3)
+    clean = _to(inp, dev)
+    want = _call(gdn_tree_chunk_update, clean, width)
+    node = 5
+    {"v": inp["v"][0, node, 1], "k": inp["k"][0, node, 0], "a": inp["a"][node]}[what][1] = float("nan")
+    g = _to(inp, dev)
+    g["records"].fill_(0.0)
+    got = _call(gdn_tree_chunk_update, g, width)
+    torch.cuda.synchronize()
+    hit = torch.zeros(len(tree), 2, 32, dtype=torch.bool, device=dev)
+    below = [node]
+    for j in range(node + 1, len(tree)):
+        if tree[j] in below:
+            below.append(j)
+    cols = {"v": (slice(1, 2), slice(1, 2)), "k": (slice(0, 2), slice(0, 32)), "a": (slice(1, 2), slice(0, 32))}[what]
+    hit[below, cols[0], cols[1]] = True
+    assert torch.equal(got[0].isnan(), hit)
+    assert torch.equal(got[0][~hit], want[0][~hit])
+    row = int(inp["record_indices"][0])
+    assert torch.equal(g["records"][row, : len(tree), :, :32].isnan(), hit)
