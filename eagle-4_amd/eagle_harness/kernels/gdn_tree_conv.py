@@ -54,12 +54,13 @@ def gdn_tree_conv1d_update(
         activation = "silu" if activation is True else None
     batch, dim, seqlen = x.shape
     width = tree_ancestors.shape[2]
+    state_len = conv_state.shape[-1]
     if query_start_loc is not None:
         assert batch == 1
         batch, seqlen = query_start_loc.shape[0] - 1, width
     assert x.element_size() == 2 and weight.element_size() == 2 and conv_state.element_size() == 2
     assert weight.shape[1] == 4 and tree_ancestors.shape[0] >= batch and tree_ancestors.shape[1:] == (3, seqlen)
-    assert tree_ancestors.is_contiguous() and conv_state.shape[-1] >= 3
+    assert tree_ancestors.is_contiguous() and state_len >= 3
     has_windows = intermediate_conv_window is not None
     if out is None:
         out = torch.empty_like(x)
@@ -69,37 +70,39 @@ def gdn_tree_conv1d_update(
     if tree_ancestors.dtype != torch.int32:
         raise _native.NotCovered("tree_ancestors must be int32")
     qsl = query_start_loc is not None
+    x_s, w_s, cs_s, o_s = x.stride(), weight.stride(), conv_state.stride(), out.stride()
+    win_s = intermediate_conv_window.stride() if has_windows else (0, 0, 0, 0)
     args = _native.ConvArgs(
         x=x.data_ptr(),
-        stride_x_seq=0 if qsl else x.stride(0),
-        stride_x_dim=x.stride(1),
-        stride_x_token=x.stride(2),
+        stride_x_seq=0 if qsl else x_s[0],
+        stride_x_dim=x_s[1],
+        stride_x_token=x_s[2],
         weight=weight.data_ptr(),
-        stride_w_dim=weight.stride(0),
-        stride_w_width=weight.stride(1),
+        stride_w_dim=w_s[0],
+        stride_w_width=w_s[1],
         bias=_native.ptr(bias),
         conv_state=conv_state.data_ptr(),
-        stride_cs_seq=conv_state.stride(0),
-        stride_cs_dim=conv_state.stride(1),
-        stride_cs_tok=conv_state.stride(2),
+        stride_cs_seq=cs_s[0],
+        stride_cs_dim=cs_s[1],
+        stride_cs_tok=cs_s[2],
         conv_state_indices=_native.itab(conv_state_indices),
         num_accepted=_native.itab(num_accepted_tokens),
         query_start_loc=_native.itab(query_start_loc),
         window=_native.ptr(intermediate_conv_window),
-        stride_win_seq=intermediate_conv_window.stride(0) if has_windows else 0,
-        stride_win_step=intermediate_conv_window.stride(1) if has_windows else 0,
-        stride_win_dim=intermediate_conv_window.stride(2) if has_windows else 0,
-        stride_win_win=intermediate_conv_window.stride(3) if has_windows else 0,
+        stride_win_seq=win_s[0],
+        stride_win_step=win_s[1],
+        stride_win_dim=win_s[2],
+        stride_win_win=win_s[3],
         window_indices=_native.itab(intermediate_state_indices if has_windows else None),
         ancestors=tree_ancestors.data_ptr(),
         out=out.data_ptr(),
-        stride_o_seq=0 if qsl else out.stride(0),
-        stride_o_dim=out.stride(1),
-        stride_o_token=out.stride(2),
+        stride_o_seq=0 if qsl else o_s[0],
+        stride_o_dim=o_s[1],
+        stride_o_token=o_s[2],
         batch=batch,
         dim=dim,
         seqlen=seqlen,
-        state_len=conv_state.shape[-1],
+        state_len=state_len,
         pad_slot_id=pad_slot_id,
         silu=1 if activation in ("silu", "swish") else 0,
         dtype=_native.dtype_code(x.dtype),

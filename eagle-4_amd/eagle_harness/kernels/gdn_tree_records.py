@@ -22,28 +22,29 @@ from eagle_harness.kernels import _native
 def _records_layout(records: torch.Tensor, HV: int, V: int, K: int) -> None:
     if records.dtype != torch.float32 or records.ndim < 4:
         raise _native.NotCovered("records must be fp32 [..., rows, steps, HV, REC]")
-    rec = records.shape[-1]
-    if (records.shape[-2] != HV or records.stride(-1) != 1 or records.stride(-2) != rec
-            or records.stride(-3) != HV * rec or rec < V + K + 1):
+    shape, strides = records.shape, records.stride()
+    rec = shape[-1]
+    if shape[-2] != HV or strides[-3:] != (HV * rec, rec, 1) or rec < V + K + 1:
         raise _native.NotCovered("each record row must be a contiguous [steps, HV, REC >= V + K + 1] block")
 
 
 def _update(A_log, dt_bias, q, k, v, a, b, state, state_indices, query_start_loc, parent, tree_paths, records,
             record_indices, width, path_replay: bool) -> torch.Tensor:
     _, tokens, H, K = k.shape
-    HV, V = v.shape[2], v.shape[3]
+    _, _, HV, V = v.shape
     N = query_start_loc.numel() - 1
     out = torch.empty_like(v)
     if N == 0 or tokens == 0:
         return out
     if width > 64:
         raise ValueError(f"tree width {width} > 64")
-    for name, t, d in (("q", q, K), ("k", k, K), ("v", v, V)):
-        if t.stride(3) != 1 or t.stride(2) != d or t.stride(1) % 4 or t.data_ptr() % (4 * t.element_size()):
+    q_s, k_s, v_s, a_s, b_s, state_s = q.stride(), k.stride(), v.stride(), a.stride(), b.stride(), state.stride()
+    for name, t, s, d in (("q", q, q_s, K), ("k", k, k_s, K), ("v", v, v_s, V)):
+        if s[3] != 1 or s[2] != d or s[1] % 4 or t.data_ptr() % (4 * t.element_size()):
             raise _native.NotCovered(f"{name} must be token-strided and contiguous over (heads, dim)")
-    if not (q.dtype == k.dtype == v.dtype) or a.dtype != b.dtype or a.stride(-1) != 1 or b.stride(-1) != 1:
+    if not (q.dtype == k.dtype == v.dtype) or a.dtype != b.dtype or a_s[-1] != 1 or b_s[-1] != 1:
         raise _native.NotCovered("q, k, v must share a dtype, as must a and b (unit stride over heads)")
-    if state.shape[1:] != (HV, V, K) or state.stride(-1) != 1 or state.stride(-2) != K or state.stride(-3) != V * K:
+    if state.shape[1:] != (HV, V, K) or state_s[1:] != (V * K, K, 1):
         raise _native.NotCovered(f"state must be a pool of contiguous [HV, V, K] = [{HV}, {V}, {K}] slots")
     _records_layout(records, HV, V, K)
     if records.shape[-3] < width:
@@ -56,13 +57,13 @@ def _update(A_log, dt_bias, q, k, v, a, b, state, state_indices, query_start_loc
         raise _native.NotCovered("parent must hold [batch, width] entries")
     args = _native.RecordsArgs(
         q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(),
-        stride_q=q.stride(1), stride_k=k.stride(1), stride_v=v.stride(1),
+        stride_q=q_s[1], stride_k=k_s[1], stride_v=v_s[1],
         in_dtype=_native.dtype_code(q.dtype), gate_dtype=_native.dtype_code(b.dtype),
-        a=a.data_ptr(), b=b.data_ptr(), stride_a=a.stride(-2), stride_b=b.stride(-2),
+        a=a.data_ptr(), b=b.data_ptr(), stride_a=a_s[-2], stride_b=b_s[-2],
         A_log=A_log.data_ptr(), dt_bias=dt_bias.data_ptr(),
         A_log_dtype=_native.dtype_code(A_log.dtype), dt_bias_dtype=_native.dtype_code(dt_bias.dtype),
         scale=K**-0.5, out_dtype=_native.dtype_code(out.dtype), out=out.data_ptr(), stride_o=out.stride(1),
-        state=state.data_ptr(), stride_state=state.stride(0), state_dtype=_native.dtype_code(state.dtype),
+        state=state.data_ptr(), stride_state=state_s[0], state_dtype=_native.dtype_code(state.dtype),
         path_replay=int(path_replay), state_indices=_native.itab(state_indices),
         query_start_loc=_native.itab(query_start_loc), parent=_native.itab(parent),
         tree_paths=_native.itab(tree_paths) if path_replay else _native.itab(None),

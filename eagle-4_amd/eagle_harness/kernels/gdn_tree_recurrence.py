@@ -28,6 +28,20 @@ from eagle_harness.kernels import _native
 from eagle_harness.kernels.gdn_tree import PAD_SLOT_ID
 
 
+def _check_state_tables(initial_state_indices: torch.Tensor, num_accepted_tokens: Optional[torch.Tensor],
+                        intermediate_states_buffer: torch.Tensor, intermediate_state_indices: torch.Tensor,
+                        publish: Optional[torch.Tensor]) -> bool:
+    """The assertions on a walk launch's state tables; True when the snapshots go to per-row slots."""
+    per_row = intermediate_state_indices.dim() == 2
+    if per_row:
+        assert intermediate_states_buffer.dim() == 4, "one slot per row addresses a [slots, HV, V, K] buffer"
+    else:
+        assert intermediate_states_buffer.dim() == 5, "one slot per request addresses a [slots, steps, HV, V, K] buffer"
+    assert (initial_state_indices.dim() == 2) == (num_accepted_tokens is not None)
+    assert publish is None or per_row, "publish copies a table of per-row slots"
+    return per_row
+
+
 def gdn_tree_state_args(
     initial_state_source: torch.Tensor,
     initial_state_indices: torch.Tensor,
@@ -44,14 +58,9 @@ def gdn_tree_state_args(
     [slots, steps, HV, V, K] scratch, sglang) selects the layout; ``num_accepted_tokens`` comes with, and only with,
     a 2-D initial-state table; ``publish`` needs per-row slots. Entries the chosen layout does not read hold a
     stride of 0, or a tensor that is safe to pass, and the flags say so."""
-    per_row = intermediate_state_indices.dim() == 2
-    if per_row:
-        assert intermediate_states_buffer.dim() == 4, "one slot per row addresses a [slots, HV, V, K] buffer"
-    else:
-        assert intermediate_states_buffer.dim() == 5, "one slot per request addresses a [slots, steps, HV, V, K] buffer"
-    h0_per_column = initial_state_indices.dim() == 2
-    assert h0_per_column == (num_accepted_tokens is not None)
-    assert publish is None or per_row, "publish copies a table of per-row slots"
+    per_row = _check_state_tables(initial_state_indices, num_accepted_tokens, intermediate_states_buffer,
+                                  intermediate_state_indices, publish)
+    h0_per_column = num_accepted_tokens is not None
 
     def inner_stride(t: torch.Tensor) -> int:  # column stride of a 2-D table; 0 for a 1-D one
         return t.stride(1) if t.dim() == 2 else 0
@@ -74,11 +83,11 @@ def gdn_tree_state_args(
 
 
 def _check_state_layout(t: torch.Tensor, lead: int, HV: int, V: int, K: int, name: str) -> None:
-    inner = t.shape[lead:]
-    if tuple(inner) != (HV, V, K) or t.stride(-1) != 1 or t.stride(-2) != K or t.stride(-3) != V * K:
+    strides = t.stride()
+    if t.shape[lead:] != (HV, V, K) or strides[lead:] != (V * K, K, 1):
         raise _native.NotCovered(f"{name}: each slot must be a contiguous [HV, V, K] = [{HV}, {V}, {K}] state")
     align = 16 if t.dtype == torch.float32 else 8
-    if t.data_ptr() % align or any(s % 4 for s in t.stride()[:lead]):
+    if t.data_ptr() % align or strides[0] % 4 or strides[lead - 1] % 4:  # one or two leading dims
         raise _native.NotCovered(f"{name}: slots must start on {align}-byte boundaries")
 
 
@@ -145,42 +154,39 @@ def gdn_tree_recurrent_update(
     fp32_state = intermediate_states_buffer.dtype == torch.float32 and initial_state_source.dtype == torch.float32
     if out is None:
         out = q.new_empty(v.shape)
-    assert out.shape == v.shape and out.stride(3) == 1 and out.stride(2) == V
+    o_s = out.stride()
+    assert out.shape == v.shape and o_s[3] == 1 and o_s[2] == V
     if tree_paths is not None and fp32_state:
         assert tree_paths.shape[0] >= N and tree_paths.dtype == torch.int32
         assert initial_state_indices.ndim == 1 and intermediate_state_indices.ndim == 1 and publish is None
         assert pad_slot_id == PAD_SLOT_ID, "the path replay takes sglang's per-request tables"
-    state = gdn_tree_state_args(
-        initial_state_source,
-        initial_state_indices,
-        num_accepted_tokens,
-        intermediate_states_buffer,
-        intermediate_state_indices,
-        publish,
-    )
+    row_slots = _check_state_tables(initial_state_indices, num_accepted_tokens, intermediate_states_buffer,
+                                    intermediate_state_indices, publish)
+    snap_s = intermediate_states_buffer.stride()
     # layouts the kernel addresses: unit inner strides, heads contiguous, 8 / 16-byte vector loads
-    for name, t, d in (("q", q, K), ("k", k, K), ("v", v, V)):
-        if t.stride(3) != 1 or t.stride(2) != d or t.stride(1) % 4 or t.data_ptr() % (4 * t.element_size()):
+    q_s, k_s, v_s, a_s, b_s = q.stride(), k.stride(), v.stride(), a.stride(), b.stride()
+    for name, t, s, d in (("q", q, q_s, K), ("k", k, k_s, K), ("v", v, v_s, V)):
+        if s[3] != 1 or s[2] != d or s[1] % 4 or t.data_ptr() % (4 * t.element_size()):
             raise _native.NotCovered(f"{name} must be token-strided and contiguous over (heads, dim)")
-    if not (q.dtype == k.dtype == v.dtype) or a.dtype != b.dtype or a.stride(-1) != 1 or b.stride(-1) != 1:
+    if not (q.dtype == k.dtype == v.dtype) or a.dtype != b.dtype or a_s[-1] != 1 or b_s[-1] != 1:
         raise _native.NotCovered("q, k, v must share a dtype, as must a and b (unit stride over heads)")
     if publish is not None and publish.dtype != torch.int32:
         raise _native.NotCovered("publish must be int32")
     _check_state_layout(initial_state_source, 1, HV, V, K, "initial_state_source")
-    _check_state_layout(intermediate_states_buffer, state["ROW_SLOTS"] and 1 or 2, HV, V, K, "intermediate_states_buffer")
+    _check_state_layout(intermediate_states_buffer, 1 if row_slots else 2, HV, V, K, "intermediate_states_buffer")
     args = _native.GdnArgs(
         q=q.data_ptr(),
         k=k.data_ptr(),
         v=v.data_ptr(),
-        stride_q=q.stride(1),
-        stride_k=k.stride(1),
-        stride_v=v.stride(1),
+        stride_q=q_s[1],
+        stride_k=k_s[1],
+        stride_v=v_s[1],
         in_dtype=_native.dtype_code(q.dtype),
         gate_dtype=_native.dtype_code(b.dtype),
         a=a.data_ptr(),
         b=b.data_ptr(),
-        stride_a=a.stride(-2),
-        stride_b=b.stride(-2),
+        stride_a=a_s[-2],
+        stride_b=b_s[-2],
         A_log=A_log.data_ptr(),
         dt_bias=dt_bias.data_ptr(),
         A_log_dtype=_native.dtype_code(A_log.dtype),
@@ -190,28 +196,28 @@ def gdn_tree_recurrent_update(
         scale=scale,
         out_dtype=_native.dtype_code(out.dtype),
         out=out.data_ptr(),
-        stride_o=out.stride(1),
+        stride_o=o_s[1],
         parents=_native.itab(retrieve_parent_token),
         cu_seqlens=_native.itab(cu_seqlens),
         h0_source=initial_state_source.data_ptr(),
-        stride_h0_source=state["stride_h0_source"],
+        stride_h0_source=initial_state_source.stride(0),
         h0_dtype=_native.dtype_code(initial_state_source.dtype),
         snap_dtype=_native.dtype_code(intermediate_states_buffer.dtype),
         h0_indices=_native.itab(initial_state_indices),
         num_accepted=_native.itab(num_accepted_tokens),
         snap=intermediate_states_buffer.data_ptr(),
-        stride_snap_slot=state["stride_snap_slot"],
-        stride_snap_row=state["stride_snap_row"],
+        stride_snap_slot=snap_s[0],
+        stride_snap_row=0 if row_slots else snap_s[1],
         snap_indices=_native.itab(intermediate_state_indices),
         publish=_native.ptr(publish),
-        stride_publish=state["stride_publish"],
-        num_slot_cols=state["num_slot_cols"],
+        stride_publish=publish.stride(0) if publish is not None else 0,
+        num_slot_cols=intermediate_state_indices.shape[-1],
         N=N,
         H=H,
         HV=HV,
         K=K,
         V=V,
-        row_slots=int(state["ROW_SLOTS"]),
+        row_slots=int(row_slots),
         skip_chain_reload=int(fp32_state),
         pad_slot_id=pad_slot_id,
     )

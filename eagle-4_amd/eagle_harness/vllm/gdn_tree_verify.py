@@ -191,12 +191,15 @@ class TreeVerify(LinearAttnVerifyExtension):
         input projection is read in place) into a new [tokens, channels] tensor. Each request's history is the conv
         state of its slot column 0, read from column ``num_accepted - 1``; the stage's window codes name each row's
         three ancestors."""
-        result = torch.empty(packed.shape, dtype=packed.dtype, device=packed.device)
-        num_reqs = rows.query_start_loc.shape[0] - 1
-        gdn_tree_conv1d_update(packed.t()[None], rows.conv_state, rows.conv_weight, rows.conv_bias, rows.activation,
-                               conv_state_indices=rows.state_indices[:, 0], intermediate_conv_window=None,
-                               intermediate_state_indices=None, tree_ancestors=stage.ancestors[:num_reqs],
-                               pad_slot_id=NULL_BLOCK_ID, out=result.t()[None],
+        tokens, channels = packed.shape
+        row, col = packed.stride()
+        result = torch.empty((tokens, channels), dtype=packed.dtype, device=packed.device)
+        # [1, channels, tokens] views in one call each: view calls were half of the layer's host time
+        gdn_tree_conv1d_update(packed.as_strided((1, channels, tokens), (0, col, row)), rows.conv_state,
+                               rows.conv_weight, rows.conv_bias, rows.activation,
+                               conv_state_indices=rows.state_indices.select(1, 0), intermediate_conv_window=None,
+                               intermediate_state_indices=None, tree_ancestors=stage.ancestors,
+                               pad_slot_id=NULL_BLOCK_ID, out=result.as_strided((1, channels, tokens), (0, 1, channels)),
                                num_accepted_tokens=rows.num_accepted_tokens, query_start_loc=rows.query_start_loc)
         return result
 
@@ -214,20 +217,23 @@ class TreeVerify(LinearAttnVerifyExtension):
         slots ``rows.state_indices`` of ``rows.ssm_state`` and its output to ``rows.out``."""
         stage = _staged()
         mixed = self._tree_conv(stage, rows, rows.mixed_qkv)
-        tokens = mixed.shape[0]
-        kdim, vdim = rows.num_k_heads * rows.head_k_dim, rows.num_v_heads * rows.head_v_dim
-        q, k, v = self._column_views(mixed, (kdim, kdim, vdim))
-        per_head = lambda t, d: t.view(1, tokens, -1, d)  # noqa: E731  [1, tokens, heads, d], token-strided
+        tokens, channels = mixed.shape
+        key_heads, dk, value_heads, dv = rows.num_k_heads, rows.head_k_dim, rows.num_v_heads, rows.head_v_dim
+        kdim = key_heads * dk
+        if channels < 2 * kdim + value_heads * dv:
+            raise ValueError(f"mixed_qkv has {channels} channels, the layer's heads make {2 * kdim + value_heads * dv}")
+        # [1, tokens, heads, d] column blocks of the conv's output, token-strided
+        heads = lambda n, d, at: mixed.as_strided((1, tokens, n, d), (0, channels, d, 1), at)  # noqa: E731
         slot_rows = rows.state_indices
         publish = stage.state_slots.get(rows.layer_name)  # set for the one layer per KV cache group that publishes
         gdn_tree_recurrent_update(
-            rows.A_log, rows.dt_bias, per_head(q, rows.head_k_dim), per_head(k, rows.head_k_dim),
-            per_head(v, rows.head_v_dim), rows.a, rows.b,
+            rows.A_log, rows.dt_bias, heads(key_heads, dk, 0), heads(key_heads, dk, kdim),
+            heads(value_heads, dv, 2 * kdim), rows.a, rows.b,
             initial_state_source=rows.ssm_state, initial_state_indices=slot_rows,
             num_accepted_tokens=rows.num_accepted_tokens, cu_seqlens=rows.query_start_loc,
             intermediate_states_buffer=rows.ssm_state, intermediate_state_indices=slot_rows,
             retrieve_parent_token=stage.parents, pad_slot_id=NULL_BLOCK_ID,
-            out=per_head(rows.out, rows.head_v_dim),
+            out=rows.out.view(1, tokens, -1, dv),
             publish=None if publish is None else publish[: slot_rows.shape[0]], gluon=True)
 
     def forward_mamba2_spec_rows(self, rows: Any) -> None:

@@ -60,7 +60,8 @@ def verify_attention(
     ValueError before anything runs. Every such call on one GPU shares that buffer: calls overlapping in time race.
     """
     num_reqs = query_start_loc.shape[0] - 1
-    heads, head_dim = q.shape[1], q.shape[2]
+    _, heads, head_dim = q.shape
+    _, page, cache_heads, _ = key_cache.shape
     fp8 = key_cache.dtype == torch.float8_e4m3fn
     if fp8 and (k_scale is None or v_scale is None):
         raise ValueError("an fp8-e4m3 cache needs k_scale and v_scale ([blocks, Hkv] fp32)")
@@ -76,30 +77,33 @@ def verify_attention(
                                  f"got {tuple(sc.shape)}")
     if block_table.dtype != torch.int32:
         raise _native.NotCovered("the block table must be int32")
-    for name, t in (("q", q), ("k_new", k_new), ("v_new", v_new), ("out", out), ("key_cache", key_cache),
-                    ("value_cache", value_cache)):
-        if t.stride(-1) != 1:
-            raise _native.NotCovered(f"{name} must have a unit stride over the head dim")
-    if masks.stride(1) != 1 or masks.dtype != torch.int64:
+    q_s, kn_s, vn_s, o_s = q.stride(), k_new.stride(), v_new.stride(), out.stride()
+    kc_s, vc_s, mask_s = key_cache.stride(), value_cache.stride(), masks.stride()
+    if not q_s[-1] == kn_s[-1] == vn_s[-1] == o_s[-1] == kc_s[-1] == vc_s[-1] == 1:
+        for name, s in (("q", q_s), ("k_new", kn_s), ("v_new", vn_s), ("out", o_s), ("key_cache", kc_s),
+                        ("value_cache", vc_s)):
+            if s[-1] != 1:
+                raise _native.NotCovered(f"{name} must have a unit stride over the head dim")
+    if mask_s[1] != 1 or masks.dtype != torch.int64:
         raise _native.NotCovered("masks must be int64 with unit row stride")
     args = _native.AttnArgs(
         q=q.data_ptr(),
-        stride_qt=q.stride(0),
-        stride_qh=q.stride(1),
+        stride_qt=q_s[0],
+        stride_qh=q_s[1],
         k_new=k_new.data_ptr(),
-        stride_knt=k_new.stride(0),
-        stride_knh=k_new.stride(1),
+        stride_knt=kn_s[0],
+        stride_knh=kn_s[1],
         v_new=v_new.data_ptr(),
-        stride_vnt=v_new.stride(0),
-        stride_vnh=v_new.stride(1),
+        stride_vnt=vn_s[0],
+        stride_vnh=vn_s[1],
         key_cache=key_cache.data_ptr(),
-        stride_kb=key_cache.stride(0),
-        stride_ks=key_cache.stride(1),
-        stride_kh=key_cache.stride(2),
+        stride_kb=kc_s[0],
+        stride_ks=kc_s[1],
+        stride_kh=kc_s[2],
         value_cache=value_cache.data_ptr(),
-        stride_vb=value_cache.stride(0),
-        stride_vs=value_cache.stride(1),
-        stride_vh=value_cache.stride(2),
+        stride_vb=vc_s[0],
+        stride_vs=vc_s[1],
+        stride_vh=vc_s[2],
         k_scale=_native.ptr(k_scale),
         stride_ksb=k_scale.stride(0) if fp8 else 0,
         stride_ksh=k_scale.stride(1) if fp8 else 0,
@@ -110,18 +114,18 @@ def verify_attention(
         context_lens=_native.itab(context_lens),
         query_start_loc=_native.itab(query_start_loc),
         masks=masks.data_ptr(),
-        stride_mask=masks.stride(0),
+        stride_mask=mask_s[0],
         out=out.data_ptr(),
-        stride_ot=out.stride(0),
-        stride_oh=out.stride(1),
+        stride_ot=o_s[0],
+        stride_oh=o_s[1],
         workspace=None,
         workspace_bytes=0,
         scale=scale,
         num_reqs=num_reqs,
         Hq=heads,
-        Hkv=key_cache.shape[2],
+        Hkv=cache_heads,
         D=head_dim,
-        page=key_cache.shape[1],
+        page=page,
         max_query_len=max_query_len,
         max_blocks=block_table.shape[1],
         dtype=_native.dtype_code(q.dtype),
