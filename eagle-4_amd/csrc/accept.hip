@@ -3,7 +3,7 @@
 //
 // The argmax is the HBM-bound part (the logits of every verify row, 2.49 GB at 8192 x 151936 bf16): one workgroup
 // per row streams it with 16-byte loads and reduces (max, first index) in registers, then across the block. The walk
-// and the tail are a few hundred bytes per request, one thread per request.
+// and the tail are a few hundred bytes per request: one wave per request.
 
 #include "common.h"
 
@@ -16,59 +16,84 @@ E4_DEV bool better(float v, int64_t i, float bv, int64_t bi) {
   return v > bv || (v == bv && i < bi);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void argmax_kernel(const eagle4_argmax_args a) {
+// One workgroup of NT threads per row, HBM-bound from about 1000 rows on (vocabulary 151936, bf16, with the tree walk:
+// 4096 rows 233 -> 189 us, 6.6 TB/s; 256 rows 74 -> 18 us, 16 rows 62 -> 12 us, where four waves a row and the search of
+// nearly every vector had bound it; 50257, 256 rows, most of them not on 16 bytes: 81 -> 11 us). A row that does not start on a 16-byte boundary (an odd vocabulary) has its first
+// elements, up to the boundary, read one by one, as the last ones past the last whole vector are.
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void argmax_kernel(const eagle4_argmax_args a) {
   using S = typename T::storage;
   const int row = blockIdx.x;
   const S* p = static_cast<const S*>(a.logits) + static_cast<int64_t>(row) * a.stride_row;
   constexpr int VEC = 16 / sizeof(S);
+  const int past = static_cast<int>(reinterpret_cast<uintptr_t>(p) % 16) / static_cast<int>(sizeof(S));
+  const int lead = past == 0 ? 0 : (VEC - past < a.vocab ? VEC - past : a.vocab);
+  const int nvec = (a.vocab - lead) / VEC;
+  const S* pv = p + lead;
+  // UNR 16-byte loads per thread and group (a thread's vectors are v, v + NT, ...; positions past the row re-read its
+  // first vector and are skipped). Nontemporal: the 2.5 GB of a large batch's logits are read once and do not churn the
+  // last-level cache (449 -> 397 us at 8192 rows).
+  typedef uint32_t u32x4n __attribute__((ext_vector_type(4)));
+  constexpr int UNR = 4;
+  auto load = [&](u32x4n (&raw)[UNR], int v0) {
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int v = v0 + u * NT;
+      raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4n*>(pv + static_cast<int64_t>(v < nvec ? v : 0) * VEC));
+    }
+  };
+  auto widen = [](const u32x4n& x, float (&f)[VEC]) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      if constexpr (sizeof(S) == 4)
+        f[i] = __uint_as_float(x[i]);
+      else
+        f[i] = T::to_f32(static_cast<S>(x[i / 2] >> (16 * (i % 2))));
+    }
+  };
+  // A thread keeps its best vector, not its best element: the vector's maximum (NaN when it holds one) against the best
+  // vector's, a handful of selects and no branch. Its first maximum is found after the loop. Searched as soon as it was
+  // found, nearly every vector of a wide workgroup was searched by some lane, and the search bound the kernel.
+  float top = -INFINITY;
+  int topv = -1;
+  u32x4n best = {0u, 0u, 0u, 0u};
+  auto take = [&](const u32x4n& x, int v) {
+    float f[VEC];
+    widen(x, f);
+    float m = f[0];
+#pragma unroll
+    for (int i = 1; i < VEC; ++i) m = __builtin_elementwise_maximum(m, f[i]);
+    if (v < nvec && (m > top || (m != m && top == top) || topv < 0)) {  // a NaN is the largest, the first one stays
+      top = m;
+      topv = v;
+      best = x;
+    }
+  };
+  for (int v0 = threadIdx.x; v0 < nvec; v0 += UNR * NT) {
+    u32x4n raw[UNR];
+    load(raw, v0);
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) take(raw[u], v0 + u * NT);
+  }
   float bv = -INFINITY;
   int64_t bi = INT64_MAX;
-  const bool aligned = (reinterpret_cast<uintptr_t>(p) % 16) == 0;
-  const int nvec = aligned ? a.vocab / VEC : 0;
-  // UNR 16-byte loads in flight per thread before any is reduced (a thread's vectors are v, v + 256, ...; positions
-  // past the row re-read its first vector and are skipped)
-  constexpr int UNR = 4;
-  for (int v0 = threadIdx.x; v0 < nvec; v0 += UNR * blockDim.x) {
-    uint4 raw[UNR];
+  if (static_cast<int>(threadIdx.x) < lead) {
+    bv = T::to_f32(p[threadIdx.x]);
+    bi = threadIdx.x;
+  }
+  if (topv >= 0) {
+    float f[VEC];
+    widen(best, f);
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int v = v0 + u * static_cast<int>(blockDim.x);
-      {  // read once, nontemporally: the 2.5 GB of logits do not churn the last-level cache (449 -> 397 us at 8192 rows)
-        typedef uint32_t u32x4n __attribute__((ext_vector_type(4)));
-        const u32x4n t =
-            __builtin_nontemporal_load(reinterpret_cast<const u32x4n*>(p + static_cast<int64_t>(v < nvec ? v : 0) * VEC));
-        raw[u] = make_uint4(t.x, t.y, t.z, t.w);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int v = v0 + u * static_cast<int>(blockDim.x);
-      const S* e = reinterpret_cast<const S*>(&raw[u]);
-      float f[VEC];
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) f[i] = T::to_f32(e[i]);
-      // the vector's max (NaN-ignoring) and sum (NaN when a NaN, or opposite infinities, is in it): only a vector
-      // that can change the thread's best — a larger value, a NaN, or the thread's first vector — is searched
-      float m = f[0], sum = f[0];
-#pragma unroll
-      for (int i = 1; i < VEC; ++i) {
-        m = fmaxf(m, f[i]);
-        sum += f[i];
-      }
-      if (v < nvec && (m > bv || sum != sum || bi == INT64_MAX)) {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-          const int64_t idx = static_cast<int64_t>(v) * VEC + i;
-          if (better(f[i], idx, bv, bi)) {
-            bv = f[i];
-            bi = idx;
-          }
-        }
+    for (int i = 0; i < VEC; ++i) {
+      const int64_t idx = lead + static_cast<int64_t>(topv) * VEC + i;
+      if (better(f[i], idx, bv, bi)) {
+        bv = f[i];
+        bi = idx;
       }
     }
   }
-  for (int64_t i = static_cast<int64_t>(nvec) * VEC + threadIdx.x; i < a.vocab; i += blockDim.x) {
+  for (int64_t i = lead + static_cast<int64_t>(nvec) * VEC + threadIdx.x; i < a.vocab; i += NT) {
     const float f = T::to_f32(p[i]);
     if (better(f, i, bv, bi)) {
       bv = f;
@@ -84,15 +109,15 @@ __global__ __launch_bounds__(256) void argmax_kernel(const eagle4_argmax_args a)
       bi = oi;
     }
   }
-  __shared__ float s_v[4];
-  __shared__ int64_t s_i[4];
+  __shared__ float s_v[NT / 64];
+  __shared__ int64_t s_i[NT / 64];
   if ((threadIdx.x & 63) == 0) {
     s_v[threadIdx.x >> 6] = bv;
     s_i[threadIdx.x >> 6] = bi;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < static_cast<int>(blockDim.x >> 6); ++w)
+    for (int w = 1; w < NT / 64; ++w)
       if (better(s_v[w], s_i[w], bv, bi)) {
         bv = s_v[w];
         bi = s_i[w];
@@ -101,8 +126,47 @@ __global__ __launch_bounds__(256) void argmax_kernel(const eagle4_argmax_args a)
   }
 }
 
-// vllm/tree_accept.py:45-83 (_tree_accept_kernel): one thread per request.
-__global__ void accept_tree_kernel(const eagle4_accept_tree_args a) {
+// vllm/tree_accept.py:45-83 (_tree_accept_kernel): one wave per request, lane r holding row r's parent, draft and
+// target (one round of loads); a step of the walk is a ballot over the rows. Latency-bound; a thread walking global
+// memory row by row waited for two loads per row looked at (16 requests of 16 rows: 17.6 -> 4 us).
+__global__ __launch_bounds__(64) void accept_tree_kernel(const eagle4_accept_tree_args a) {
+  const int b = blockIdx.x, lane = threadIdx.x;
+  const int64_t slot = e4::ld(a.idx_mapping, b);
+  const int64_t start = e4::ld(a.cu_num_logits, b);
+  const int64_t rows = e4::ld(a.cu_num_logits, b + 1) - start;
+  const int limit = static_cast<int>(rows < a.width ? rows : a.width);
+  int64_t parent = -1, draft = 0, target = 0;
+  if (lane < limit) {
+    parent = e4::ld(a.parents, slot, lane);
+    draft = e4::ld(a.drafted, start + lane);
+    target = e4::ld(a.target, start + lane);
+  }
+  int node = 0, count = 0, mine = 0;  // lane s: the node of step s
+  int64_t mine_token = 0;
+  for (int step = 0; step < a.width && limit > 0; ++step) {
+    const int64_t token = __shfl(target, node);
+    if (lane == step) {
+      mine = node;
+      mine_token = token;
+    }
+    ++count;
+    // the lowest-index row that continues the walk (:78-79)
+    const uint64_t next = __ballot(lane >= 1 && lane < limit && parent == node && draft == token);
+    if (next == 0) break;
+    node = __builtin_ctzll(next);
+  }
+  if (lane < count) {
+    a.sampled[b * a.stride_sampled + lane] = mine_token;
+    a.path[slot * a.stride_path + lane] = mine;
+  }
+  if (lane == 0) {
+    a.num_sampled[b] = count;
+    a.path_len[slot] = count;
+  }
+}
+
+// The same for tables wider than a wave: one thread per request.
+__global__ void accept_wide_tree_kernel(const eagle4_accept_tree_args a) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= a.num_reqs) return;
   const int64_t slot = e4::ld(a.idx_mapping, b);
@@ -237,6 +301,18 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(const eagle4_compact_
   }
 }
 
+// 16 waves on rows of 200 KB and more, 8 on shorter ones, whose 16 waves would spend more on their own reduction than on
+// the row (bf16, us with the tree walk, 8 / 16 waves: vocabulary 151936, 16 rows 12.3 / 11.7, 256 rows 18.7 / 18.3, 4096
+// rows 193 / 189; 50257, 16 rows 9.1 / 9.3, 4096 rows 69 / 72; 32000, 4096 rows 45 / 55). 4 waves were slower in all.
+template <typename T>
+int launch_argmax(const eagle4_argmax_args& a, hipStream_t s) {
+  if (static_cast<int64_t>(a.vocab) * static_cast<int64_t>(sizeof(typename T::storage)) >= 200 * 1024)
+    argmax_kernel<T, 1024><<<a.rows, 1024, 0, s>>>(a);
+  else
+    argmax_kernel<T, 512><<<a.rows, 512, 0, s>>>(a);
+  return E4_LAUNCH_STATUS();
+}
+
 bool tab_ok(const eagle4_itab& t) { return t.ptr != nullptr && e4::is_index_dtype(t.dtype); }
 
 }  // namespace
@@ -246,12 +322,11 @@ extern "C" int eagle4_argmax_rows(const eagle4_argmax_args* a, void* stream) {
   if (a->vocab < 1 || a->out == nullptr) return EAGLE4_NOT_COVERED;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   switch (a->dtype) {
-    case EAGLE4_BF16: argmax_kernel<e4::Bf16><<<a->rows, 256, 0, s>>>(*a); break;
-    case EAGLE4_F16: argmax_kernel<e4::F16><<<a->rows, 256, 0, s>>>(*a); break;
-    case EAGLE4_F32: argmax_kernel<e4::F32><<<a->rows, 256, 0, s>>>(*a); break;
+    case EAGLE4_BF16: return launch_argmax<e4::Bf16>(*a, s);
+    case EAGLE4_F16: return launch_argmax<e4::F16>(*a, s);
+    case EAGLE4_F32: return launch_argmax<e4::F32>(*a, s);
     default: return EAGLE4_NOT_COVERED;
   }
-  return E4_LAUNCH_STATUS();
 }
 
 extern "C" int eagle4_accept_tree(const eagle4_accept_tree_args* a, void* stream) {
@@ -259,7 +334,11 @@ extern "C" int eagle4_accept_tree(const eagle4_accept_tree_args* a, void* stream
   if (!tab_ok(a->target) || !tab_ok(a->drafted) || !tab_ok(a->cu_num_logits) || !tab_ok(a->idx_mapping) ||
       !tab_ok(a->parents) || a->width < 1)
     return EAGLE4_NOT_COVERED;
-  accept_tree_kernel<<<e4::ceil_div(a->num_reqs, 64), 64, 0, static_cast<hipStream_t>(stream)>>>(*a);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (a->width <= 64)
+    accept_tree_kernel<<<a->num_reqs, 64, 0, s>>>(*a);
+  else
+    accept_wide_tree_kernel<<<e4::ceil_div(a->num_reqs, 64), 64, 0, s>>>(*a);
   return E4_LAUNCH_STATUS();
 }
 
