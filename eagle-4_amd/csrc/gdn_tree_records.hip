@@ -409,74 +409,215 @@ int launch_records(const eagle4_records_args& a, hipStream_t s) {
 }
 
 // ---- commit ------------------------------------------------------------------------------------------------------
-// 4 waves x 8 rows: one (32-row V tile, request x value head, layer) per workgroup; lane layout as in the walk.
-template <int K, int C, typename Tpool>
+// Two fp32 values rounded through the pool dtype (nearest even), as a store and a reload give.
+template <typename T>
+E4_DEV uint32_t pack_pool(float x0, float x1) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  if constexpr (T::code == EAGLE4_BF16)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), f16x2));
+}
+
+// One workgroup folds RPT x 4 x (64 / C) V rows of one (request x value head, layer): 4 waves, C lanes per row, a lane
+// holding 16-byte chunks of its rows (an 8-byte one at the smallest K). HBM-bound: the pool state once each way. What
+// kept it from that was a chain of round trips per workgroup, the path's parents one by one and then each node's record
+// as it was folded; now there are three: the tables with the parents (a lane per node), then the state with the records
+// of up to NST path nodes (staged in LDS, shared by all rows), then the store. 16 requests, 12 layers of 48 heads,
+// K = V = 128, bf16 pool: 188 -> 112 us, 5.8 TB/s (122 with regular stores: the states' next reader comes a forward
+// pass later, so they are loaded and stored nontemporally).
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t u32x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int K, int C, int RPT, typename Tpool>
 __global__ __launch_bounds__(256) void gdn_records_commit_kernel(const eagle4_records_commit_args a) {
-  constexpr int E = K / C;
-  constexpr int NJ = E / 4;
-  constexpr int ROWS = 4 * (64 / C);
   using PS = typename Tpool::storage;
-  __shared__ int s_path[64];
-  __shared__ int s_len;
+  constexpr bool kF32 = sizeof(PS) == 4;
+  constexpr int E = K / C;                             // elements per lane and row
+  constexpr int VEC = kF32 ? 4 : (E >= 8 ? 8 : 4);     // elements per chunk
+  constexpr int NJ = E / VEC;
+  constexpr int WORDS = VEC * static_cast<int>(sizeof(PS)) / 4;
+  constexpr int RW = 64 / C;                           // rows of a wave side by side
+  constexpr int ROWS = 4 * RW * RPT;
+  constexpr int NST = 16;                              // path nodes staged at a time
+  constexpr int KQ = K / 4;
+  constexpr int K_IT = (NST * KQ + 255) / 256, D_IT = (NST * ROWS + 255) / 256;
+  __shared__ __align__(16) float s_key[NST][K];
+  __shared__ float s_del[NST][ROWS];
+  __shared__ float s_eg[NST];
   const int nh = blockIdx.y, layer = blockIdx.z;
   const int n = nh / a.HV, hv = nh % a.HV;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int c = lane % C, rr = lane / C;
-  const int row = blockIdx.x * ROWS + wave * (64 / C) + rr;
-  const int64_t step = e4::ld(a.commit_steps, n), slot = e4::ld(a.state_indices, n), rrow = e4::ld(a.record_indices, n);
+  const int row0 = blockIdx.x * ROWS;
+  const int wrow = wave * RW * RPT + rr;               // the lane's first row within the workgroup, then every RW
+
+  const int64_t step = uni64(e4::ld(a.commit_steps, n)), slot = uni64(e4::ld(a.state_indices, n)),
+                rrow = uni64(e4::ld(a.record_indices, n));
+  const int up = static_cast<int>(e4::ld(a.parent, n, lane < a.dmax ? lane : 0));
   if (!(step >= 0 && slot >= 0 && rrow >= 0)) return;
-  if (tid == 0) {  // the root path, accepted node first (:192-201)
-    int node = static_cast<int>(step), len = 0;
-    for (int j = 0; j < a.dmax && j < 64 && node >= 0 && node < a.dmax; ++j) {
-      s_path[len++] = node;
-      node = node > 0 ? static_cast<int>(e4::ld(a.parent, n, node)) : -1;
-    }
-    s_len = len;
-  }
-  __syncthreads();
-  const int len = s_len;
-  PS* st = static_cast<PS*>(a.state) + layer * a.stride_state_layer + slot * a.stride_state_slot +
-           static_cast<int64_t>(hv) * a.V * K + static_cast<int64_t>(row < a.V ? row : 0) * K;
-  const float* rec = a.records + layer * a.stride_records_layer + rrow * a.stride_records_row;
-  float h[E];
+
+  // the state, in flight while the path and its records are looked up
+  PS* st[RPT];
+  uint32_t raw[RPT][NJ][WORDS];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) load4<Tpool>(st + 4 * c + 4 * C * j, &h[4 * j]);
-  for (int d = 0; d < len; ++d) {
-    const float* r = rec + (static_cast<int64_t>(s_path[len - 1 - d]) * a.HV + hv) * a.rec;
-    const float eg = r[a.V + K];
-    const float delta = r[row < a.V ? row : 0];
-    if (a.round_state && d > 0) {
-#pragma unroll
-      for (int e = 0; e < E; ++e) h[e] = e4::round_through<Tpool>(h[e]);
-    }
+  for (int s = 0; s < RPT; ++s) {
+    const int row = row0 + wrow + s * RW;
+    st[s] = static_cast<PS*>(a.state) + layer * a.stride_state_layer + slot * a.stride_state_slot +
+            (static_cast<int64_t>(hv) * a.V + (row < a.V ? row : 0)) * K + VEC * c;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
+      if constexpr (WORDS == 4) {
+        const u32x4_a8 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4_a8*>(st[s] + VEC * C * j));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float key = r[a.V + 4 * c + 4 * C * j + e];
-        h[4 * j + e] = h[4 * j + e] * eg + key * delta;
+        for (int i = 0; i < 4; ++i) raw[s][j][i] = x[i];
+      } else {
+        const u32x2_a8 x = __builtin_nontemporal_load(reinterpret_cast<const u32x2_a8*>(st[s] + VEC * C * j));
+        raw[s][j][0] = x[0];
+        raw[s][j][1] = x[1];
       }
     }
   }
-  if (row < a.V) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) store4<Tpool>(st + 4 * c + 4 * C * j, &h[4 * j]);
+  // the root path, accepted node first (:192-201); lane d keeps its d-th node
+  int path = 0, len = 0;
+  for (int node = static_cast<int>(step); len < a.dmax && len < 64 && node >= 0 && node < a.dmax;) {
+    if (lane == len) path = node;
+    ++len;
+    node = node == 0 ? -1 : node < 64 ? readlane(up, node) : static_cast<int>(uni64(e4::ld(a.parent, n, node)));
   }
+
+  const float* rec = a.records + layer * a.stride_records_layer + rrow * a.stride_records_row + static_cast<int64_t>(hv) * a.rec;
+  const int64_t node_stride = static_cast<int64_t>(a.HV) * a.rec;
+  float h[RPT][E];
+  for (int base = 0; base < len; base += NST) {  // from the root: the d-th node folded is path entry len - 1 - d
+    const int m = len - base < NST ? len - base : NST;
+    u32x4_a4 kq[K_IT];
+    float dq[D_IT], eq = 0.f;
+#pragma unroll
+    for (int it = 0; it < K_IT; ++it) {
+      const int i = tid + 256 * it, d = i / KQ;
+      const int node = __shfl(path, len - 1 - (base + (d < m ? d : 0)));
+      if (d < m) kq[it] = *reinterpret_cast<const u32x4_a4*>(rec + node * node_stride + a.V + 4 * (i % KQ));
+    }
+#pragma unroll
+    for (int it = 0; it < D_IT; ++it) {
+      const int i = tid + 256 * it, d = i / ROWS, row = row0 + i % ROWS;
+      const int node = __shfl(path, len - 1 - (base + (d < m ? d : 0)));
+      if (d < m) dq[it] = rec[node * node_stride + (row < a.V ? row : 0)];
+    }
+    {
+      const int node = __shfl(path, len - 1 - (base + (tid < m ? tid : 0)));
+      if (tid < m) eq = rec[node * node_stride + a.V + K];
+    }
+    if (base > 0) __syncthreads();  // the strip before is folded
+#pragma unroll
+    for (int it = 0; it < K_IT; ++it) {
+      const int i = tid + 256 * it, d = i / KQ;
+      if (d < m) *reinterpret_cast<u32x4*>(&s_key[d][4 * (i % KQ)]) = kq[it];
+    }
+#pragma unroll
+    for (int it = 0; it < D_IT; ++it) {
+      const int i = tid + 256 * it, d = i / ROWS;
+      if (d < m) s_del[d][i % ROWS] = dq[it];
+    }
+    if (tid < m) s_eg[tid] = eq;
+    __syncthreads();
+    if (base == 0) {
+#pragma unroll
+      for (int s = 0; s < RPT; ++s)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            if constexpr (kF32)
+              h[s][VEC * j + e] = __uint_as_float(raw[s][j][e]);
+            else
+              h[s][VEC * j + e] = Tpool::to_f32(static_cast<PS>(raw[s][j][e / 2] >> (16 * (e % 2))));
+          }
+    }
+    for (int d = 0; d < m; ++d) {
+      const float eg = s_eg[d];
+      float del[RPT];
+#pragma unroll
+      for (int s = 0; s < RPT; ++s) del[s] = s_del[d][wrow + s * RW];
+      const bool round = a.round_state && base + d > 0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        float key[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; e += 4) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(&s_key[d][VEC * c + VEC * C * j + e]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) key[e + i] = x[i];
+        }
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+          if constexpr (!kF32) {
+            if (round) {
+#pragma unroll
+              for (int e = 0; e < VEC; e += 2) {
+                const uint32_t w = pack_pool<Tpool>(h[s][VEC * j + e], h[s][VEC * j + e + 1]);
+                h[s][VEC * j + e] = Tpool::to_f32(static_cast<PS>(w));
+                h[s][VEC * j + e + 1] = Tpool::to_f32(static_cast<PS>(w >> 16));
+              }
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) h[s][VEC * j + e] = h[s][VEC * j + e] * eg + key[e] * del[s];
+        }
+      }
+    }
+  }
+  if (len == 0) return;  // a node outside the tables: the state stays
+#pragma unroll
+  for (int s = 0; s < RPT; ++s) {
+    if (row0 + wrow + s * RW >= a.V) continue;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      uint32_t w[WORDS];
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i) {
+        if constexpr (kF32)
+          w[i] = __float_as_uint(h[s][VEC * j + i]);
+        else
+          w[i] = pack_pool<Tpool>(h[s][VEC * j + 2 * i], h[s][VEC * j + 2 * i + 1]);
+      }
+      if constexpr (WORDS == 4)
+        __builtin_nontemporal_store((u32x4_a8{w[0], w[1], w[2], w[3]}), reinterpret_cast<u32x4_a8*>(st[s] + VEC * C * j));
+      else
+        __builtin_nontemporal_store((u32x2_a8{w[0], w[1]}), reinterpret_cast<u32x2_a8*>(st[s] + VEC * C * j));
+    }
+  }
+}
+
+template <int K, int C, int RPT, typename Tpool>
+int launch_commit_rows(const eagle4_records_commit_args& a, hipStream_t s) {
+  const dim3 grid(e4::ceil_div(a.V, 4 * (64 / C) * RPT), a.n * a.HV, a.layers);
+  gdn_records_commit_kernel<K, C, RPT, Tpool><<<grid, 256, 0, s>>>(a);
+  return E4_LAUNCH_STATUS();
+}
+
+// Two rows a lane once that still gives two workgroups per CU, one below (us at 1 / 2 rows, 48 heads, bf16: 16 requests of
+// 12 layers 122 / 112, 64 of 4 layers 167 / 152; 768 workgroups, 8 requests of 4 layers, 12 heads, fp32 12.5 / 10.0; 192
+// workgroups, 2 requests of 12 layers, 8 heads 5.6 / 6.1; 1 request of 1 layer 4.5 / 5.1). Four rows were slower.
+template <int K, int C, typename Tpool>
+int launch_commit_pool(const eagle4_records_commit_args& a, hipStream_t s) {
+  constexpr int ROWS2 = 8 * (64 / C);
+  if constexpr (K >= 64)
+    if (a.V >= ROWS2 && static_cast<int64_t>(e4::ceil_div(a.V, ROWS2)) * a.n * a.HV * a.layers >= 512)
+      return launch_commit_rows<K, C, 2, Tpool>(a, s);
+  return launch_commit_rows<K, C, 1, Tpool>(a, s);
 }
 
 template <int K, int C>
 int launch_commit(const eagle4_records_commit_args& a, hipStream_t s) {
-  constexpr int ROWS = 4 * (64 / C);
-  const dim3 grid(e4::ceil_div(a.V, ROWS), a.n * a.HV, a.layers);
-  if (a.state_dtype == EAGLE4_F32)
-    gdn_records_commit_kernel<K, C, e4::F32><<<grid, 256, 0, s>>>(a);
-  else if (a.state_dtype == EAGLE4_BF16)
-    gdn_records_commit_kernel<K, C, e4::Bf16><<<grid, 256, 0, s>>>(a);
-  else if (a.state_dtype == EAGLE4_F16)
-    gdn_records_commit_kernel<K, C, e4::F16><<<grid, 256, 0, s>>>(a);
-  else
-    return EAGLE4_NOT_COVERED;
-  return E4_LAUNCH_STATUS();
+  if (a.state_dtype == EAGLE4_F32) return launch_commit_pool<K, C, e4::F32>(a, s);
+  if (a.state_dtype == EAGLE4_BF16) return launch_commit_pool<K, C, e4::Bf16>(a, s);
+  if (a.state_dtype == EAGLE4_F16) return launch_commit_pool<K, C, e4::F16>(a, s);
+  return EAGLE4_NOT_COVERED;
 }
 
 }  // namespace
