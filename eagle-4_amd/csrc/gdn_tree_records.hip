@@ -242,9 +242,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_records_walk_kernel(const eagl
   auto round_h = [&]() {
     if constexpr (!kPoolExact) {
 #pragma unroll
-      for (int s = 0; s < RPT; ++s)
-#pragma unroll
-        for (int e = 0; e < E; ++e) h[s][e] = e4::round_through<Tpool>(h[s][e]);
+      for (int s = 0; s < RPT; ++s) e4::round_all<Tpool>(h[s]);
     }
   };
   // The state of node p by replaying its root path from the pool state (a parent the stack had no room for).
@@ -339,11 +337,11 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_records_walk_kernel(const eagl
           for (int s = 0; s < RPT; ++s)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-              float4 w = make_float4(h[s][4 * j], h[s][4 * j + 1], h[s][4 * j + 2], h[s][4 * j + 3]);
-              if (round)
-                w = make_float4(e4::round_through<Tpool>(w.x), e4::round_through<Tpool>(w.y),
-                                e4::round_through<Tpool>(w.z), e4::round_through<Tpool>(w.w));
-              my_stack[sp][s * NJ + j][lane] = w;
+              float w[4] = {h[s][4 * j], h[s][4 * j + 1], h[s][4 * j + 2], h[s][4 * j + 3]};
+              if constexpr (!kPoolExact) {
+                if (round) e4::round_all<Tpool>(w);
+              }
+              my_stack[sp][s * NJ + j][lane] = make_float4(w[0], w[1], w[2], w[3]);
             }
           ++sp;
         } else {
@@ -409,18 +407,6 @@ int launch_records(const eagle4_records_args& a, hipStream_t s) {
 }
 
 // ---- commit ------------------------------------------------------------------------------------------------------
-// Two fp32 values rounded through the pool dtype (nearest even), as a store and a reload give.
-template <typename T>
-E4_DEV uint32_t pack_pool(float x0, float x1) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-  if constexpr (T::code == EAGLE4_BF16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
-  else
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), f16x2));
-}
-
 // One workgroup folds RPT x 4 x (64 / C) V rows of one (request x value head, layer): 4 waves, C lanes per row, a lane
 // holding 16-byte chunks of its rows (an 8-byte one at the smallest K). HBM-bound: the pool state once each way. What
 // kept it from that was a chain of round trips per workgroup, the path's parents one by one and then each node's record
@@ -559,7 +545,7 @@ __global__ __launch_bounds__(256) void gdn_records_commit_kernel(const eagle4_re
             if (round) {
 #pragma unroll
               for (int e = 0; e < VEC; e += 2) {
-                const uint32_t w = pack_pool<Tpool>(h[s][VEC * j + e], h[s][VEC * j + e + 1]);
+                const uint32_t w = Tpool::pack(h[s][VEC * j + e], h[s][VEC * j + e + 1]);
                 h[s][VEC * j + e] = Tpool::to_f32(static_cast<PS>(w));
                 h[s][VEC * j + e + 1] = Tpool::to_f32(static_cast<PS>(w >> 16));
               }
@@ -583,7 +569,7 @@ __global__ __launch_bounds__(256) void gdn_records_commit_kernel(const eagle4_re
         if constexpr (kF32)
           w[i] = __float_as_uint(h[s][VEC * j + i]);
         else
-          w[i] = pack_pool<Tpool>(h[s][VEC * j + 2 * i], h[s][VEC * j + 2 * i + 1]);
+          w[i] = Tpool::pack(h[s][VEC * j + 2 * i], h[s][VEC * j + 2 * i + 1]);
       }
       if constexpr (WORDS == 4)
         __builtin_nontemporal_store((u32x4_a8{w[0], w[1], w[2], w[3]}), reinterpret_cast<u32x4_a8*>(st[s] + VEC * C * j));

@@ -323,11 +323,9 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
         for (int s = 0; s < RPT; ++s)
 #pragma unroll
           for (int j = 0; j < NJ; ++j) {
-            float4 w = make_float4(h[s][4 * j], h[s][4 * j + 1], h[s][4 * j + 2], h[s][4 * j + 3]);
-            if constexpr (!kExact)
-              w = make_float4(e4::round_through<Tsnap>(w.x), e4::round_through<Tsnap>(w.y),
-                              e4::round_through<Tsnap>(w.z), e4::round_through<Tsnap>(w.w));
-            my_stack[sp][s * NJ + j][lane] = w;
+            float w[4] = {h[s][4 * j], h[s][4 * j + 1], h[s][4 * j + 2], h[s][4 * j + 3]};
+            if constexpr (!kExact) e4::round_all<Tsnap>(w);
+            my_stack[sp][s * NJ + j][lane] = make_float4(w[0], w[1], w[2], w[3]);
           }
         ++sp;
       } else {
@@ -338,9 +336,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
       if constexpr (!kExact) {
         if (!(a.skip_chain_reload && next == u + 1)) {  // an fp32 chain child keeps the registers
 #pragma unroll
-          for (int s = 0; s < RPT; ++s)
-#pragma unroll
-            for (int e = 0; e < E; ++e) h[s][e] = e4::round_through<Tsnap>(h[s][e]);
+          for (int s = 0; s < RPT; ++s) e4::round_all<Tsnap>(h[s]);
         }
       }
     } else {

@@ -36,8 +36,8 @@ E4_DEV void store4(typename T::storage* p, const float* in) {
     *reinterpret_cast<f32x4v*>(p) = f32x4v{in[0], in[1], in[2], in[3]};
   } else {
     u32x2v v;
-    v.x = static_cast<uint32_t>(T::from_f32(in[0])) | (static_cast<uint32_t>(T::from_f32(in[1])) << 16);
-    v.y = static_cast<uint32_t>(T::from_f32(in[2])) | (static_cast<uint32_t>(T::from_f32(in[3])) << 16);
+    v.x = T::pack(in[0], in[1]);
+    v.y = T::pack(in[2], in[3]);
     *reinterpret_cast<u32x2v*>(p) = v;
   }
 }
@@ -53,8 +53,7 @@ E4_DEV void store4_buf(__amdgpu_buffer_rsrc_t r, int byte_off, const float* in) 
     const u32x4v v = {__float_as_uint(in[0]), __float_as_uint(in[1]), __float_as_uint(in[2]), __float_as_uint(in[3])};
     __builtin_amdgcn_raw_buffer_store_b128(v, r, byte_off, 0, AUX);
   } else {
-    const u32x2v v = {static_cast<uint32_t>(T::from_f32(in[0])) | (static_cast<uint32_t>(T::from_f32(in[1])) << 16),
-                      static_cast<uint32_t>(T::from_f32(in[2])) | (static_cast<uint32_t>(T::from_f32(in[3])) << 16)};
+    const u32x2v v = {T::pack(in[0], in[1]), T::pack(in[2], in[3])};
     __builtin_amdgcn_raw_buffer_store_b64(v, r, byte_off, 0, AUX);
   }
 }

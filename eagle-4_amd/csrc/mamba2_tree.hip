@@ -61,14 +61,20 @@ E4_DEV f32x4 load4(const typename S::storage* p) {
   }
 }
 
+// v rounded through a 16-bit storage dtype
+template <typename S>
+E4_DEV f32x4 round4(f32x4 v) {
+  float w[4] = {v.x, v.y, v.z, v.w};
+  e4::round_all<S>(w);
+  return f32x4{w[0], w[1], w[2], w[3]};
+}
+
 template <typename S>
 E4_DEV void store4(typename S::storage* p, f32x4 v) {
   if constexpr (sizeof(typename S::storage) == 4) {
     *reinterpret_cast<f32x4*>(p) = v;
   } else {
-    const uint32_t lo = S::from_f32(v.x) | (static_cast<uint32_t>(S::from_f32(v.y)) << 16);
-    const uint32_t hi = S::from_f32(v.z) | (static_cast<uint32_t>(S::from_f32(v.w)) << 16);
-    *reinterpret_cast<u32x2*>(p) = u32x2{lo, hi};
+    *reinterpret_cast<u32x2*>(p) = u32x2{S::pack(v.x, v.y), S::pack(v.z, v.w)};
   }
 }
 
@@ -256,9 +262,7 @@ __global__ __launch_bounds__(NT) void mamba2_tree_kernel(const eagle4_mamba2_arg
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               f32x4 w = st[j];
-              if constexpr (!kExact)
-                w = f32x4{e4::round_through<S>(w.x), e4::round_through<S>(w.y), e4::round_through<S>(w.z),
-                          e4::round_through<S>(w.w)};
+              if constexpr (!kExact) w = round4<S>(w);
               my_stack[sp][j][lane] = w;
             }
             ++sp;
@@ -270,9 +274,7 @@ __global__ __launch_bounds__(NT) void mamba2_tree_kernel(const eagle4_mamba2_arg
           if constexpr (!kExact) {
             if (next != u + 1) {  // not the chain child: it starts from the stored (rounded) state
 #pragma unroll
-              for (int j = 0; j < 4; ++j)
-                st[j] = f32x4{e4::round_through<S>(st[j].x), e4::round_through<S>(st[j].y),
-                              e4::round_through<S>(st[j].z), e4::round_through<S>(st[j].w)};
+              for (int j = 0; j < 4; ++j) st[j] = round4<S>(st[j]);
             }
           }
         } else {
