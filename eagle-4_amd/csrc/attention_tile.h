@@ -2,6 +2,8 @@
 // of a K / V tile, the MFMA operand reads, and one online-softmax step of a wave's 16 query rows.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace e4attn {
@@ -13,7 +15,7 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));  // a 16-byte MFMA operand as a native vector
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 
-// Splits whose partials a merge thread loads at once (the split-schedule, fp32 and draft-row merges).
+// Splits whose partials a merge thread loads at once.
 constexpr int kMergeGroup = 8;
 constexpr int kTileKeys = 32;
 
@@ -243,6 +245,83 @@ struct StreamPlan {
   int seg_cost;  // a segment's end in quarter tiles, for the cost-weighted shares
   int64_t part_off, lse_off;  // float offsets into the workspace (the int64 prefix of tiles per request is first)
 };
+
+// Merges the n normalised fp32 partials of one row by their log2-sum-exps: weights 2^(lse_i - max). The partials are rows
+// part_of(i) of part_out [., D] and lse [.]; a thread takes four columns, D / 4 adjacent threads a row, and SG such runs
+// share a row, run j folding the partials j, j + SG, ..., kMergeGroup of them in flight. A row of many partials is a chain
+// of round trips, which SG shortens (one request, 8 query heads of D 64 over 129 splits, SG 16: 52 -> 6.3 us; 16
+// heads of D 128 over 43 splits, SG 8: 20 -> 4.4 us). Up to kMergeGroup partials and SG 1 the operations and their
+// order are those of a sum over all partials with one maximum. Every thread of the workgroup calls it (n 0 where it has
+// no row); true in the run that holds the row's sum and weight sum.
+template <int D, int SG, typename PartOf>
+E4_DEV bool merge_partials(int n, PartOf part_of, const float* part_out, const float* lse, f32x4_t& sum, float& wsum) {
+  constexpr int LP = D / 4;
+  const int run = threadIdx.x / LP, sub = run % SG, d = 4 * (threadIdx.x % LP);
+  float top = -INFINITY;
+  sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  wsum = 0.f;
+  for (int s0 = sub; s0 < n; s0 += SG * kMergeGroup) {
+    float l[kMergeGroup];
+    f32x4_t v[kMergeGroup];
+#pragma unroll
+    for (int i = 0; i < kMergeGroup; ++i) {  // past the last partial: the group's first again, not used
+      const int64_t part = part_of(s0 + SG * i < n ? s0 + SG * i : s0);
+      l[i] = lse[part];
+      v[i] = *reinterpret_cast<const f32x4_t*>(part_out + part * D + d);
+    }
+    float now = top;
+#pragma unroll
+    for (int i = 0; i < kMergeGroup; ++i)
+      if (s0 + SG * i < n) now = fmaxf(now, l[i]);
+    const float keep = top == -INFINITY ? 0.f : exp2f(top - now);
+    sum *= keep;
+    wsum *= keep;
+    top = now;
+#pragma unroll
+    for (int i = 0; i < kMergeGroup; ++i) {
+      if (s0 + SG * i >= n || l[i] == -INFINITY) continue;  // a partial without a visible key weighs nothing
+      const float w = exp2f(l[i] - top);
+      sum += w * v[i];
+      wsum += w;
+    }
+  }
+  if constexpr (SG > 1) {
+    __shared__ f32x4_t s_sum[256];
+    __shared__ float2 s_top[256 / LP];
+    s_sum[threadIdx.x] = sum;
+    if (d == 0) s_top[run] = make_float2(top, wsum);
+    __syncthreads();
+    if (sub != 0) return false;
+    float all = top;
+#pragma unroll
+    for (int j = 1; j < SG; ++j) all = fmaxf(all, s_top[run + j].x);
+    const float keep = top == -INFINITY ? 0.f : exp2f(top - all);
+    sum *= keep;
+    wsum *= keep;
+#pragma unroll
+    for (int j = 1; j < SG; ++j) {
+      const float2 o = s_top[run + j];
+      if (o.x == -INFINITY && o.y == 0.f) continue;
+      const float w = exp2f(o.x - all);
+      sum += w * s_sum[threadIdx.x + LP * j];
+      wsum += w * o.y;
+    }
+  }
+  return true;
+}
+
+// The runs per row for rows of about `partials` each, `rows` rows in all: one where a thread takes them in one round trip,
+// else as many as a workgroup holds (up to 16) or four, as long as that makes fewer than 2048 workgroups (from there on
+// starting them costs more than the round trips: 64 segments of 96 rows over 5 pieces at D 256, 6144 workgroups of four
+// runs 15.6 us, 9.7 without). `go` gets the number as a type tag.
+template <int D, typename F>
+int with_merge_runs(int64_t partials, int64_t rows, F&& go) {
+  constexpr int kMost = 1024 / D < 16 ? 1024 / D : 16;
+  const auto groups = [&](int runs) { return rows * runs * (D / 4) / 256; };
+  if (partials > 4 * kMergeGroup && groups(kMost) < 2048) return go(std::integral_constant<int, kMost>{});
+  if (partials > kMergeGroup && groups(4) < 2048) return go(std::integral_constant<int, 4>{});
+  return go(std::integral_constant<int, 1>{});
+}
 
 // One request whose block table holds at most 4096 keys is too small for the streamed schedule's per-workgroup setup
 // (~10 us of table loads, share search and ring fill before the first tile): the split schedule with 96-key splits

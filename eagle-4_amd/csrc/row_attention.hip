@@ -215,53 +215,25 @@ __global__ __launch_bounds__(NT) void row_attention_kernel(const eagle4_row_attn
   }
 }
 
-// _merge_splits_kernel (:202-224): D / 4 lanes per (row, query head), 4 consecutive columns each (16-byte loads of
-// the partials), 256 / (D / 4) pairs per workgroup; weights 2^(lse - max) over the splits.
-template <int D, typename T>
+// _merge_splits_kernel (:202-224): the splits of each (row, query head) merged.
+template <int D, int SG, typename T>
 __global__ __launch_bounds__(256) void row_merge_kernel(const eagle4_row_attn_args a, int splits) {
-  constexpr int LP = D / 4, PAIRS = 256 / LP;
-  const int64_t pair = static_cast<int64_t>(blockIdx.x) * PAIRS + threadIdx.x / LP;
+  constexpr int LP = D / 4, PAIRS = 256 / LP / SG;
+  const int64_t pair = static_cast<int64_t>(blockIdx.x) * PAIRS + threadIdx.x / (LP * SG);
   const int d = 4 * (threadIdx.x % LP);
-  if (pair >= static_cast<int64_t>(a.bs) * a.rows_per_request * a.heads) return;
+  const bool ok = pair < static_cast<int64_t>(a.bs) * a.rows_per_request * a.heads;
   const int64_t row = pair / a.heads;
   const int head = static_cast<int>(pair % a.heads);
   const int64_t b = row / a.rows_per_request, t = row % a.rows_per_request;
   const int64_t part0 = ((b * a.heads + head) * (a.splits + 1)) * a.rows_padded + t;
-  // The splits in groups of kMergeGroup, every load of a group issued before the first is used (one memory round trip
-  // per group, not per split; a group's loads past the last split re-read the first), the same operations in the same
-  // order as one split at a time.
-  float top = -INFINITY;
-  for (int s0 = 0; s0 < splits; s0 += kMergeGroup) {
-    float l[kMergeGroup];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) l[i] = a.part_lse[part0 + (s0 + i < splits ? s0 + i : s0) * a.rows_padded];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i)
-      if (s0 + i < splits) top = fmaxf(top, l[i]);
-  }
-  float wsum = 0.f;
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < splits; s0 += kMergeGroup) {
-    float l[kMergeGroup];
-    f32x4_t v[kMergeGroup];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) {
-      const int64_t part = part0 + (s0 + i < splits ? s0 + i : s0) * a.rows_padded;
-      l[i] = a.part_lse[part];
-      v[i] = *reinterpret_cast<const f32x4_t*>(a.part_out + part * D + d);
-    }
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) {
-      if (s0 + i >= splits) break;
-      const float w = l[i] == -INFINITY ? 0.f : exp2f(l[i] - top);
-      wsum += w;
-      if (w != 0.f) acc += w * v[i];
-    }
-  }
+  f32x4_t acc;
+  float wsum;
+  const bool mine = merge_partials<D, SG>(ok ? splits : 0,
+                                          [&](int i) { return part0 + static_cast<int64_t>(i) * a.rows_padded; },
+                                          a.part_out, a.part_lse, acc, wsum);
+  if (!mine || !ok) return;
   uint16_t* o = static_cast<uint16_t*>(a.out) + row * a.stride_o_row + static_cast<int64_t>(head) * a.stride_o_head + d;
-  const uint32_t lo = T::from_f32(acc.x / wsum) | (static_cast<uint32_t>(T::from_f32(acc.y / wsum)) << 16);
-  const uint32_t hi = T::from_f32(acc.z / wsum) | (static_cast<uint32_t>(T::from_f32(acc.w / wsum)) << 16);
-  *reinterpret_cast<uint2*>(o) = make_uint2(lo, hi);
+  *reinterpret_cast<uint2*>(o) = make_uint2(T::pack(acc.x / wsum, acc.y / wsum), T::pack(acc.z / wsum, acc.w / wsum));
 }
 
 template <int D, typename T>
@@ -270,9 +242,13 @@ int launch(const eagle4_row_attn_args& a, hipStream_t s) {
   const int groups = (R + 16 * NW - 1) / (16 * NW);
   const int splits = a.splits + (a.step == 0 ? 0 : 1);
   row_attention_kernel<D, T><<<dim3(splits, a.kv_heads * groups, a.bs), NT, 0, s>>>(a, groups);
-  const int64_t pairs = static_cast<int64_t>(a.bs) * a.rows_per_request * a.heads, per = 256 / (D / 4);
-  row_merge_kernel<D, T><<<static_cast<unsigned>((pairs + per - 1) / per), 256, 0, s>>>(a, splits);
-  return E4_LAUNCH_STATUS();
+  const int64_t pairs = static_cast<int64_t>(a.bs) * a.rows_per_request * a.heads;
+  return with_merge_runs<D>(splits, pairs, [&](auto runs) {
+    constexpr int SG = decltype(runs)::value;
+    constexpr int64_t per = 256 / (D / 4) / SG;
+    row_merge_kernel<D, SG, T><<<static_cast<unsigned>((pairs + per - 1) / per), 256, 0, s>>>(a, splits);
+    return E4_LAUNCH_STATUS();
+  });
 }
 
 template <typename T>

@@ -310,64 +310,30 @@ __global__ __launch_bounds__(64 * NW) void verify_attention_kernel(const eagle4_
   }
 }
 
-// vllm/verify_attention.py:115-139 (_verify_merge_kernel) for the requests with more than one split: one thread per
-// 4 consecutive d of a row.
-template <int D, typename T>
+// vllm/verify_attention.py:115-139 (_verify_merge_kernel) for the requests with more than one split.
+template <int D, int SG, typename T>
 __global__ __launch_bounds__(256) void verify_merge_kernel(const eagle4_attn_args a, int chunk, int row_tiles,
                                                            int max_splits) {
   const int b = blockIdx.z, kvh = blockIdx.y;
   const Req rq = request_info(a, b, chunk);
   if (rq.splits <= 1) return;
   constexpr int TPR = D / 4;
-  const int rho = blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  const int rho = blockIdx.x * (256 / TPR / SG) + threadIdx.x / (TPR * SG);
   const int d = 4 * (threadIdx.x % TPR);
   const int G = a.Hq / a.Hkv;
   const int t = rho / G, gq = rho % G;
   const int rows = row_tiles * 16;
-  if (rho >= rows || t >= rq.width) return;
+  const bool ok = rho < rows && t < rq.width;
   const float* lse = a.workspace + static_cast<int64_t>(a.num_reqs) * a.Hkv * max_splits * rows * D;
   const int64_t part0 = (static_cast<int64_t>(b) * a.Hkv + kvh) * max_splits * rows + rho;
-  // The splits in groups of kMergeGroup, every load of a group issued before the first is used (one memory round trip
-  // per group, not per split; a group's loads past the last split re-read the first), the same operations in the same
-  // order as one split at a time.
-  const int ns = rq.splits;
-  float mx = -INFINITY;
-  for (int s0 = 0; s0 < ns; s0 += kMergeGroup) {
-    float l[kMergeGroup];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) l[i] = lse[part0 + static_cast<int64_t>(s0 + i < ns ? s0 + i : s0) * rows];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i)
-      if (s0 + i < ns) mx = fmaxf(mx, l[i]);
-  }
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-  float wsum = 0.f;
-  for (int s0 = 0; s0 < ns; s0 += kMergeGroup) {
-    float l[kMergeGroup];
-    float4 v[kMergeGroup];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) {
-      const int64_t part = part0 + static_cast<int64_t>(s0 + i < ns ? s0 + i : s0) * rows;
-      l[i] = lse[part];
-      v[i] = *reinterpret_cast<const float4*>(a.workspace + part * D + d);
-    }
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) {
-      if (s0 + i >= ns) break;
-      const float w = l[i] == -INFINITY ? 0.f : exp2f(l[i] - mx);
-      sum.x += w * v[i].x;
-      sum.y += w * v[i].y;
-      sum.z += w * v[i].z;
-      sum.w += w * v[i].w;
-      wsum += w;
-    }
-  }
+  f32x4_t sum;
+  float wsum;
+  const bool mine = merge_partials<D, SG>(ok ? rq.splits : 0, [&](int i) { return part0 + static_cast<int64_t>(i) * rows; },
+                                          a.workspace, lse, sum, wsum);
+  if (!mine || !ok) return;
   const float inv = 1.0f / wsum;
   uint16_t* op = static_cast<uint16_t*>(a.out) + (rq.start + t) * a.stride_ot + (static_cast<int64_t>(kvh) * G + gq) * a.stride_oh + d;
-  uint2 w;
-  w.x = static_cast<uint32_t>(T::from_f32(sum.x * inv)) | (static_cast<uint32_t>(T::from_f32(sum.y * inv)) << 16);
-  w.y = static_cast<uint32_t>(T::from_f32(sum.z * inv)) | (static_cast<uint32_t>(T::from_f32(sum.w * inv)) << 16);
-  *reinterpret_cast<uint2*>(op) = w;
+  *reinterpret_cast<uint2*>(op) = make_uint2(T::pack(sum.x * inv, sum.y * inv), T::pack(sum.z * inv, sum.w * inv));
 }
 
 struct Plan {
@@ -422,9 +388,12 @@ int launch(const eagle4_attn_args& a, const Plan& p, hipStream_t s) {
   const dim3 grid(p.max_splits, a.Hkv * p.row_groups, a.num_reqs);
   verify_attention_kernel<D, NW, T, FP8><<<grid, 64 * NW, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
   if (p.max_splits > 1) {
-    constexpr int RPB = 256 / (D / 4);
-    const dim3 mgrid(e4::ceil_div(p.row_tiles * 16, RPB), a.Hkv, a.num_reqs);
-    verify_merge_kernel<D, T><<<mgrid, 256, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
+    return with_merge_runs<D>(p.max_splits, int64_t(p.row_tiles) * 16 * a.Hkv * a.num_reqs, [&](auto runs) {
+      constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
+      const dim3 mgrid(e4::ceil_div(p.row_tiles * 16, RPB), a.Hkv, a.num_reqs);
+      verify_merge_kernel<D, SG, T><<<mgrid, 256, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
+      return E4_LAUNCH_STATUS();
+    });
   }
   return E4_LAUNCH_STATUS();
 }

@@ -226,61 +226,27 @@ __global__ __launch_bounds__(64 * kTilesF) void verify_f32_kernel(const eagle4_a
   }
 }
 
-// The splits of a row merged (vllm/verify_attention.py:115-139): weights 2^(lse_s - max) over the normalised
-// partials; one thread per 4 consecutive d of a row.
-template <int D>
+// The splits of a row merged (vllm/verify_attention.py:115-139).
+template <int D, int SG>
 __global__ __launch_bounds__(256) void verify_f32_merge(const eagle4_attn_args a, int chunk, int row_tiles,
                                                         int max_splits) {
   constexpr int TPR = D / 4;
-  constexpr int RPB = 256 / TPR;
   const int b = blockIdx.z, kvh = blockIdx.y;
   const ReqF rq = req_f(a, b, chunk);
   if (rq.splits <= 1 || rq.width <= 0) return;
-  const int rho = blockIdx.x * RPB + threadIdx.x / TPR, d = 4 * (threadIdx.x % TPR);
+  const int rho = blockIdx.x * (256 / TPR / SG) + threadIdx.x / (TPR * SG), d = 4 * (threadIdx.x % TPR);
   const int G = a.Hq / a.Hkv;
   const int rows = rq.width < a.max_query_len ? rq.width : a.max_query_len;
   const int t = rho / G, gq = rho % G;
-  if (rho >= row_tiles * 16 || t >= rows) return;
   const int nrow = row_tiles * 16;
+  const bool ok = rho < nrow && t < rows;
   const float* lse = a.workspace + static_cast<int64_t>(a.num_reqs) * a.Hkv * max_splits * nrow * D;
   const int64_t part0 = (static_cast<int64_t>(b) * a.Hkv + kvh) * max_splits * nrow + rho;
-  // The splits in groups of kMergeGroup, every load of a group issued before the first is used (one memory round trip
-  // per group, not per split; a group's loads past the last split re-read the first), the same operations in the same
-  // order as one split at a time.
-  const int ns = rq.splits;
-  float mx = -INFINITY;
-  for (int s0 = 0; s0 < ns; s0 += kMergeGroup) {
-    float l[kMergeGroup];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i) l[i] = lse[part0 + static_cast<int64_t>(s0 + i < ns ? s0 + i : s0) * nrow];
-#pragma unroll
-    for (int i = 0; i < kMergeGroup; ++i)
-      if (s0 + i < ns) mx = fmaxf(mx, l[i]);
-  }
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-  float wsum = 0.f;
-  if (mx != -INFINITY) {
-    for (int s0 = 0; s0 < ns; s0 += kMergeGroup) {
-      float l[kMergeGroup];
-      float4 v[kMergeGroup];
-#pragma unroll
-      for (int i = 0; i < kMergeGroup; ++i) {
-        const int64_t part = part0 + static_cast<int64_t>(s0 + i < ns ? s0 + i : s0) * nrow;
-        l[i] = lse[part];
-        v[i] = *reinterpret_cast<const float4*>(a.workspace + part * D + d);
-      }
-#pragma unroll
-      for (int i = 0; i < kMergeGroup; ++i) {
-        if (s0 + i >= ns) break;
-        const float w = exp2f(l[i] - mx);
-        sum.x += w * v[i].x;
-        sum.y += w * v[i].y;
-        sum.z += w * v[i].z;
-        sum.w += w * v[i].w;
-        wsum += w;
-      }
-    }
-  }
+  f32x4_t sum;
+  float wsum;
+  const bool mine = merge_partials<D, SG>(ok ? rq.splits : 0, [&](int i) { return part0 + static_cast<int64_t>(i) * nrow; },
+                                          a.workspace, lse, sum, wsum);
+  if (!mine || !ok) return;
   const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
   *reinterpret_cast<float4*>(static_cast<float*>(a.out) + (rq.start + t) * a.stride_ot +
                              (static_cast<int64_t>(kvh) * G + gq) * a.stride_oh + d) =
@@ -310,9 +276,12 @@ int launch_f(const eagle4_attn_args& a, const PlanF& p, hipStream_t s) {
   const dim3 grid(p.max_splits, a.Hkv * p.row_groups, a.num_reqs);
   verify_f32_kernel<D><<<grid, 64 * kTilesF, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
   if (p.max_splits > 1) {
-    constexpr int RPB = 256 / (D / 4);
-    const dim3 mgrid(e4::ceil_div(p.row_tiles * 16, RPB), a.Hkv, a.num_reqs);
-    verify_f32_merge<D><<<mgrid, 256, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
+    return with_merge_runs<D>(p.max_splits, int64_t(p.row_tiles) * 16 * a.Hkv * a.num_reqs, [&](auto runs) {
+      constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
+      const dim3 mgrid(e4::ceil_div(p.row_tiles * 16, RPB), a.Hkv, a.num_reqs);
+      verify_f32_merge<D, SG><<<mgrid, 256, 0, s>>>(a, p.chunk, p.row_tiles, p.max_splits);
+      return E4_LAUNCH_STATUS();
+    });
   }
   return E4_LAUNCH_STATUS();
 }

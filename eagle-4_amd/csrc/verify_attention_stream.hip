@@ -1204,6 +1204,37 @@ __global__ __launch_bounds__(256) void verify_stream_merge(const eagle4_attn_arg
   }
 }
 
+// The same for segments cut into many pieces (a few long requests over the whole grid): a thread takes four columns and
+// SG runs of threads share a row.
+template <int D, int SG, typename T>
+__global__ __launch_bounds__(256) void verify_stream_merge_many(const eagle4_attn_args a, const StreamPlan p) {
+  constexpr int TPR = D / 4;
+  const int s = blockIdx.x;
+  const int b = s / p.HR, k = s - b * p.HR;
+  const int64_t* pre = reinterpret_cast<const int64_t*>(a.workspace);
+  if (pre[b + 1] - pre[b] <= 0) return;
+  const int32_t* const seg_w = reinterpret_cast<const int32_t*>(pre + a.num_reqs + 1) + 2 * static_cast<int64_t>(s);
+  const int w0 = seg_w[0], w1 = seg_w[1];
+  if (w0 == w1) return;  // inside one share: written directly
+  const int r = blockIdx.y * (256 / TPR / SG) + threadIdx.x / (TPR * SG), d = 4 * (threadIdx.x % TPR);
+  const int rows_seg = p.rows_seg, G = p.G, kvh = k / p.RG, rg = k - kvh * p.RG;
+  const int64_t qs = e4::ld(a.query_start_loc, b);
+  int64_t rows = e4::ld(a.query_start_loc, b + 1) - qs;
+  rows = rows < a.max_query_len ? rows : a.max_query_len;
+  const int rho = rg * rows_seg + r, t = rho / G, gq = rho - t * G;
+  const bool ok = r < rows_seg && rho / 16 < p.row_tiles && t < rows;
+  f32x4_t sum;
+  float wsum;
+  const bool mine = merge_partials<D, SG>(
+      ok ? w1 - w0 + 1 : 0,
+      [&](int i) { return static_cast<int64_t>(i == 0 ? 2 * w0 + 1 : 2 * (w0 + i)) * rows_seg + r; },
+      a.workspace + p.part_off, a.workspace + p.lse_off, sum, wsum);
+  if (!mine || !ok) return;
+  const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
+  uint16_t* o = static_cast<uint16_t*>(a.out) + (qs + t) * a.stride_ot + (static_cast<int64_t>(kvh) * G + gq) * a.stride_oh + d;
+  *reinterpret_cast<uint2*>(o) = make_uint2(T::pack(sum.x * inv, sum.y * inv), T::pack(sum.z * inv, sum.w * inv));
+}
+
 template <int D, int C, typename T, bool FP8>
 int resident_groups() {
   static const int per_cu = [] {
@@ -1224,11 +1255,20 @@ int resident_groups() {
 template <int D, int C, typename T, bool FP8>
 int launch(const eagle4_attn_args& a, const StreamPlan& p, hipStream_t s) {
   verify_stream_kernel<D, C, T, FP8><<<p.nwg, 64 * (C + kProducers), 0, s>>>(a, p);
+  // Segments of many pieces (shares per segment, on average) fold them in parallel; from five on that is faster if the rows
+  // leave room for more runs (1 request of 16384 keys, 4 KV heads at D 128: 129 pieces 35 -> 6.3 us; 4 of 2048 keys 8.5 ->
+  // 5.5 us; 16 of 1024 keys at D 64, 9 pieces 6.2 -> 4.4 us).
+  const int64_t segs = static_cast<int64_t>(a.num_reqs) * p.HR, pieces = p.nwg / segs + 1;
   constexpr int kMergeThreadsPerRow = D / (D < 16 ? D : 16);
-  verify_stream_merge<D, T><<<dim3(a.num_reqs * p.HR,
-                                   e4::ceil_div(static_cast<int64_t>(p.rows_seg) * kMergeThreadsPerRow, 256)),
-                              256, 0, s>>>(a, p);
-  return E4_LAUNCH_STATUS();
+  return with_merge_runs<D>(pieces > 4 ? pieces + kMergeGroup : 1, segs * p.rows_seg, [&](auto runs) {
+    constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
+    if constexpr (SG > 1)
+      verify_stream_merge_many<D, SG, T><<<dim3(segs, e4::ceil_div(p.rows_seg, RPB)), 256, 0, s>>>(a, p);
+    else
+      verify_stream_merge<D, T><<<dim3(segs, e4::ceil_div(static_cast<int64_t>(p.rows_seg) * kMergeThreadsPerRow, 256)),
+                                  256, 0, s>>>(a, p);
+    return E4_LAUNCH_STATUS();
+  });
 }
 
 // The instantiations: head dims 32 .. 256, 2 / 4 / 6 consumer waves (a group of row tiles takes the smallest that
