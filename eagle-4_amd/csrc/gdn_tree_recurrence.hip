@@ -58,7 +58,7 @@ E4_DEV void item_of(int id, int HV, int tiles, int& n, int& hv, int& tile) {
 // The request's first TS nodes are staged in LDS up front (q, k, the workgroup's v rows, and the node scalars), so the
 // walk itself issues no global loads for them: a vector load in the walk would wait for the snapshot stores before it
 // (loads and stores share the vmcnt counter), which serialises the walk on the store latency.
-template <int K, int C, int RPT, int WAVES, int S, bool SMALL, typename Tin, typename Tsnap>
+template <int K, int C, int RPT, int WAVES, int S, bool SMALL, int STAGED, typename Tin, typename Tsnap>
 __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_gdn_args a) {
   constexpr int E = K / C;
   constexpr int NJ = E / 4;
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
   static_assert(E % 4 == 0 && C <= 64, "lane layout");
   using IS = typename Tin::storage;
   using SS = typename Tsnap::storage;
-  constexpr int TS = sizeof(IS) == 4 ? 8 : 16;  // staged nodes
+  constexpr int TS = sizeof(IS) == 4 ? STAGED / 2 : STAGED;  // staged nodes
   constexpr bool kExact = sizeof(SS) == 4;      // fp32 snapshots: a reload gives the registers bit for bit
   constexpr bool kFastWalk = E <= 8;            // the depth-first walk of staged nodes has a loop of its own
   // The parked-state stack; in the prologue, before any state is parked, it holds the staged nodes' raw q and k rows.
@@ -186,7 +186,10 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
   const int plan = ps.plan[lane];  // read before the walk writes s_out (after the next barrier)
   const bool dfs = ps.dfs != 0;
   // L2 norms over K (:143-151) and q^, k^ (read by every node of the walk) in one pass
-  stage_norms<Tin, K, TS, NT>(s_qr, s_kr, s_sc, ts, tid, a.scale, s_q, s_k);
+  if (STAGED > 16 && ts <= TS / 2)  // twice the threads a node
+    stage_norms<Tin, K, TS, NT, TS / 2>(s_qr, s_kr, s_sc, ts, tid, a.scale, s_q, s_k);
+  else
+    stage_norms<Tin, K, TS, NT>(s_qr, s_kr, s_sc, ts, tid, a.scale, s_q, s_k);
   __syncthreads();  // the raw rows' space becomes the stack
 
   settle_loads();  // the initial state and the plan tables
@@ -460,26 +463,26 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
   }
 }
 
-template <int K, int C, int RPT, int WAVES, int S, bool SMALL, typename Tin>
+template <int K, int C, int RPT, int WAVES, int S, bool SMALL, int STAGED, typename Tin>
 int launch_snap(const eagle4_gdn_args& a, hipStream_t s) {
   constexpr int ROWS = WAVES * RPT * (64 / C);
   const dim3 grid(e4::ceil_div(a.V, ROWS) * a.HV * a.N);
   if (a.snap_dtype == EAGLE4_F32)
-    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, Tin, e4::F32><<<grid, 64 * WAVES, 0, s>>>(a);
+    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, STAGED, Tin, e4::F32><<<grid, 64 * WAVES, 0, s>>>(a);
   else if (a.snap_dtype == EAGLE4_BF16)
-    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, Tin, e4::Bf16><<<grid, 64 * WAVES, 0, s>>>(a);
+    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, STAGED, Tin, e4::Bf16><<<grid, 64 * WAVES, 0, s>>>(a);
   else if (a.snap_dtype == EAGLE4_F16)
-    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, Tin, e4::F16><<<grid, 64 * WAVES, 0, s>>>(a);
+    gdn_tree_walk_kernel<K, C, RPT, WAVES, S, SMALL, STAGED, Tin, e4::F16><<<grid, 64 * WAVES, 0, s>>>(a);
   else
     return EAGLE4_NOT_COVERED;
   return E4_LAUNCH_STATUS();
 }
 
-template <int K, int C, int RPT, int WAVES, int S, bool SMALL = false>
+template <int K, int C, int RPT, int WAVES, int S, bool SMALL = false, int STAGED = 16>
 int launch_in(const eagle4_gdn_args& a, hipStream_t s) {
-  if (a.in_dtype == EAGLE4_BF16) return launch_snap<K, C, RPT, WAVES, S, SMALL, e4::Bf16>(a, s);
-  if (a.in_dtype == EAGLE4_F16) return launch_snap<K, C, RPT, WAVES, S, SMALL, e4::F16>(a, s);
-  if (a.in_dtype == EAGLE4_F32) return launch_snap<K, C, RPT, WAVES, S, SMALL, e4::F32>(a, s);
+  if (a.in_dtype == EAGLE4_BF16) return launch_snap<K, C, RPT, WAVES, S, SMALL, STAGED, e4::Bf16>(a, s);
+  if (a.in_dtype == EAGLE4_F16) return launch_snap<K, C, RPT, WAVES, S, SMALL, STAGED, e4::F16>(a, s);
+  if (a.in_dtype == EAGLE4_F32) return launch_snap<K, C, RPT, WAVES, S, SMALL, STAGED, e4::F32>(a, s);
   return EAGLE4_NOT_COVERED;
 }
 
@@ -513,7 +516,22 @@ extern "C" int eagle4_gdn_tree_recurrent_update(const eagle4_gdn_args* a, void* 
       // jumping, then a pass per tree level): they walk children in index order and park up to four states instead
       // of two, enough for the nesting of index order in drafted trees (a parent beyond them reloads its snapshot),
       // and store their snapshots nontemporally.
-      if (groups8 <= 256) return launch_in<128, 16, 1, 4, 4, true>(*a, s);
+      // Trees of more than 16 rows (known here only from a per-row slot table's columns) have 32 nodes staged instead of
+      // 16: a node past the staged ones is loaded in the walk, where its loads wait for every snapshot store in flight. On
+      // the small grids always (1 request of 32 nodes, 32 heads, fp32 53.7 -> 29.6 us; 16 nodes under a 32-column table
+      // 19.5 us both ways). The larger ones pay with a third of their workgroups per CU, so there from the widths on
+      // where it was faster (layer, us, 16 / 32 staged: fp32 4 requests of 24 rows 64.5 / 61.6, 16 of 24 rows 175 / 174,
+      // 64 of 24 rows 654 / 684, 64 of 32 rows 941 / 928; bf16 4 of 20 rows 47 / 41, 64 of 17 rows 317 / 363, 64 of 24
+      // rows 567 / 475, 64 of 32 rows 818 / 601).
+      const int cols = a->row_slots ? a->num_slot_cols : 0;
+      const bool exact = a->snap_dtype == EAGLE4_F32;
+      const bool wide = groups8 <= 256    ? cols > 16
+                        : groups8 <= 1024 ? cols >= (exact ? 24 : 20)
+                        : groups8 <= 2048 ? cols >= 24
+                                          : cols >= (exact ? 30 : 24);
+      if (groups8 <= 256)
+        return wide ? launch_in<128, 16, 1, 4, 4, true, 32>(*a, s) : launch_in<128, 16, 1, 4, 4, true>(*a, s);
+      if (wide) return launch_in<128, 8, 1, 4, 2, false, 32>(*a, s);
       return launch_in<128, 8, 1, 4, 2>(*a, s);
     }
     case 256: return launch_in<256, 16, 1, 4, 2>(*a, s);

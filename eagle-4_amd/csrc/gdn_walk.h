@@ -256,12 +256,12 @@ struct Staging {
 // adjacent threads share a node, each summing a contiguous run of its q and k; .z = scale / |q|, .w = 1 / |k|
 // (1e-6 inside the square roots). With qh / kh, every thread also writes its run of q^ = q .z and k^ = k .w there
 // (the same products the separate pass makes), so no second pass over the raw rows follows.
-template <typename Tin, int K, int TS, int NT>
+template <typename Tin, int K, int TS, int NT, int NODES = TS>
 E4_DEV void stage_norms(const typename Tin::storage (&s_q)[TS][K], const typename Tin::storage (&s_k)[TS][K],
                         float4 (&s_sc)[TS], int ts, int tid, float scale, float (*qh)[K] = nullptr,
                         float (*kh)[K] = nullptr) {
-  constexpr int LPN0 = NT / TS < 64 ? NT / TS : 64;
-  constexpr int LPN = LPN0 < K ? LPN0 : K;  // threads per node (a power of two)
+  constexpr int LPN0 = NT / NODES < 64 ? NT / NODES : 64;
+  constexpr int LPN = LPN0 < K ? LPN0 : K;  // threads per node (a power of two); NODES >= ts
   constexpr int PER = K / LPN;                       // elements each
   static_assert(PER >= 1 && K % LPN == 0, "norm split");
   const int t = tid / LPN, part = tid % LPN;
