@@ -39,7 +39,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int WAVES = 4;          // waves per workgroup
 constexpr int NT = 64 * WAVES;    // threads per workgroup
-constexpr int ROWS = 16 * WAVES;  // V rows per workgroup
 
 // The pool dtype's arithmetic: the MFMA over raw 16-bit operands, widening of the low / high element of a word, and
 // the packed fp32 -> 16-bit conversion (round to nearest even: what a store to the pool dtype and a reload give).
@@ -167,10 +166,13 @@ E4_DEV void chain_walk(const eagle4_records_args& a, int64_t bos, int Tn, int id
 }
 
 // One workgroup: V rows [tile ROWS, (tile + 1) ROWS) of one (request, value head); WMAX >= width staged nodes; S
-// parked states per wave.
-template <int K, int WMAX, int S, typename T>
+// parked states per wave; RT 16-row tiles per wave, which share the walk's steps, the children's lists and scalars and, at
+// V = 128, one staging of the head's rows. Trees of 17 to 32 nodes in 32 staged rows, not 64, which left one workgroup per
+// CU: 32 requests of 32 nodes, 48 heads 316 -> 175 us, with two tiles a wave 127 us.
+template <int K, int WMAX, int S, int RT, typename T>
 __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_args a, int tiles, int per_xcd,
                                                          int total) {
+  constexpr int ROWS = 16 * WAVES * RT;  // V rows per workgroup
   constexpr int KB = K / 32;    // MFMA blocks over K
   constexpr int KQ = K / 4;     // K elements per lane group
   constexpr int CHK = K / 8;    // 16-byte chunks per q / k row
@@ -200,8 +202,10 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   const int ih = hv / (a.HV / a.H);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   const int row0 = tile * ROWS;
-  const int wrow = wave * 16 + r16;            // the lane's row within the workgroup
-  const bool wave_on = row0 + wave * 16 < a.V;  // V % 16 == 0: a wave's rows are all inside or all past V
+  const int wrow = wave * 16 * RT + r16;       // the lane's row of its first tile, within the workgroup; the others + 16 i
+  // V % 16 == 0: a tile's rows are all inside or all past V
+  const int left = (a.V - row0) / 16 - wave * RT, tiles_on = left < 0 ? 0 : left < RT ? left : RT;
+  const bool wave_on = tiles_on > 0;
 
   const int64_t bos = uni64(e4::ld(a.query_start_loc, n));
   const int T_ = static_cast<int>(uni64(e4::ld(a.query_start_loc, n + 1)) - bos);
@@ -213,7 +217,8 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   const float A = -expf(widen_raw(A_raw, a.A_log_dtype));
   const float dt_bias = widen_raw(dt_raw, a.dt_bias_dtype);
   if (rec_row < 0) {  // a request without records never reloads a parent: one chain, no rounding
-    if (wave_on) chain_walk<K, T>(a, bos, T_, idx, hv, ih, row0 + wave * 16, lane, A, dt_bias);
+    for (int i = 0; i < tiles_on; ++i)
+      chain_walk<K, T>(a, bos, T_, idx, hv, ih, row0 + (wave * RT + i) * 16, lane, A, dt_bias);
     return;
   }
   const int Tn = T_ < a.width ? T_ : a.width;  // a tree has at most width (<= WMAX) rows
@@ -223,16 +228,18 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   // slot index (zeros: the zero initial state, :73-75) or a wave past V
   const char* h0_base = static_cast<const char*>(a.state) +
                         ((idx >= 0 ? static_cast<int64_t>(idx) * a.stride_state : 0) +
-                         (static_cast<int64_t>(hv) * a.V + row0 + wave * 16) * K) * 2;
+                         (static_cast<int64_t>(hv) * a.V + row0 + wave * 16 * RT) * K) * 2;
   const __amdgpu_buffer_rsrc_t h0_rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(h0_base), 0, idx >= 0 && wave_on ? 16 * K * 2 : 0, 0x00020000);
-  auto load_h0 = [&](u32x4 (&Hc)[KB]) {
+      const_cast<char*>(h0_base), 0, idx >= 0 ? tiles_on * 16 * K * 2 : 0, 0x00020000);
+  auto load_h0 = [&](u32x4 (&Hc)[RT][KB]) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-      Hc[kb] = __builtin_bit_cast(u32x4,
-                                  __builtin_amdgcn_raw_buffer_load_b128(h0_rs, (r16 * K + g * KQ + 8 * kb) * 2, 0, 0));
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        Hc[i][kb] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(h0_rs, ((16 * i + r16) * K + g * KQ + 8 * kb) * 2, 0, 0));
   };
-  u32x4 H[KB];
+  u32x4 H[RT][KB];
   load_h0(H);
   u32x4 kr[QK_IT], qr[QK_IT];
   uint16_t vr[V_IT];
@@ -392,60 +399,71 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   // The children of node u (-1: the roots) from its rounded state Hc, eight per pass: one MFMA pass gives h~ k_j
   // (operand rows 0-7) and h~ q_j (rows 8-15); lane (g, r16) receives element r of row 4 g + r for V row r16, i.e.
   // h~ k (g < 2) or h~ q (g >= 2) of child 4 (g % 2) + r of the pass.
-  auto serve = [&](int u, int nch, const u32x4 (&Hc)[KB]) {
+  auto serve = [&](int u, int nch, const u32x4 (&Hc)[RT][KB]) {
     for (int base = 0; base < nch; base += 8) {
       const uint8_t* list = &s_ch[u + 1][base];
       const int mine = list[r16 & 7];  // the child whose k (r16 < 8) or q this lane's operand row holds
       const uint32_t cw = *reinterpret_cast<const uint32_t*>(list + 4 * (g & 1));  // the lane's 4 result children
       int c[4];
       float4 nd[4];
-      float vv[4];
+      float vv[RT][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int x = (cw >> (8 * r)) & 0xff;
         c[r] = x == 0xff ? -1 : x;
         const int cc = x == 0xff ? 0 : x;
         nd[r] = s_nd[cc];
-        vv[r] = O::lo(s_v[cc][wrow]);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) vv[i][r] = O::lo(s_v[cc][wrow + 16 * i]);
       }
       const uint16_t* src = (r16 < 8 ? &s_k[0][0] : &s_q[0][0]) + (mine == 0xff ? 0 : mine) * PITCH + g * KQ;
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+      f32x4_t acc[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         u32x4 x = *reinterpret_cast<const u32x4*>(src + 8 * kb);
         if (mine == 0xff) x = u32x4{0u, 0u, 0u, 0u};
-        acc = O::mma(x, Hc[kb], acc);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i] = O::mma(x, Hc[i][kb], acc[i]);
       }
       // lanes g < 2: delta = (v - decay ks h~ k) beta; lanes g >= 2: decay qs h~ q (the output less delta ks qs k.q)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = g < 2 ? (vv[r] - nd[r].x * acc[r]) * nd[r].y : nd[r].z * acc[r];
-        if (c[r] >= 0) (g < 2 ? s_dv : s_oq)[c[r]][wrow] = x;
-      }
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const float x = g < 2 ? (vv[i][r] - nd[r].x * acc[i][r]) * nd[r].y : nd[r].z * acc[i][r];
+          if (c[r] >= 0) (g < 2 ? s_dv : s_oq)[c[r]][wrow + 16 * i] = x;
+        }
     }
     lds_order();
   };
   // Hc <- round(decay_j Hc + k^_j delta_j^T): node j's rounded state from its parent's
-  auto advance = [&](u32x4 (&Hc)[KB], int j) {
+  auto advance = [&](u32x4 (&Hc)[RT][KB], int j) {
     const float decay = s_gk[j].x;
-    const float dv = s_dv[j][wrow];
+    float dv[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) dv[i] = s_dv[j][wrow + 16 * i];
     const float* kp = &s_kh[j][g * KQ];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const float4 k0 = *reinterpret_cast<const float4*>(kp + 8 * kb);
       const float4 k1 = *reinterpret_cast<const float4*>(kp + 8 * kb + 4);
       const float kh[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-      uint32_t nw[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t hw = Hc[kb][e];
-        nw[e] = O::pack(fmaf(kh[2 * e], dv, O::lo(hw) * decay), fmaf(kh[2 * e + 1], dv, O::hi(hw) * decay));
+      for (int i = 0; i < RT; ++i) {
+        uint32_t nw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t hw = Hc[i][kb][e];
+          nw[e] = O::pack(fmaf(kh[2 * e], dv[i], O::lo(hw) * decay), fmaf(kh[2 * e + 1], dv[i], O::hi(hw) * decay));
+        }
+        Hc[i][kb] = u32x4{nw[0], nw[1], nw[2], nw[3]};
       }
-      Hc[kb] = u32x4{nw[0], nw[1], nw[2], nw[3]};
     }
   };
 
-  u32x4 st[S][KB];
+  u32x4 st[S][RT][KB];
   int sid[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) sid[s] = -3;
@@ -454,11 +472,15 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
 #pragma unroll
     for (int s = S - 1; s > 0; --s) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) st[s][kb] = st[s - 1][kb];
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) st[s][i][kb] = st[s - 1][i][kb];
       sid[s] = sid[s - 1];
     }
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) st[0][kb] = H[kb];
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) st[0][i][kb] = H[i][kb];
     sid[0] = u;
     sp = sp < S ? sp + 1 : S;
   };
@@ -467,7 +489,9 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
 #pragma unroll
     for (int s = 0; s + 1 < S; ++s) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) st[s][kb] = st[s + 1][kb];
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) st[s][i][kb] = st[s + 1][i][kb];
       sid[s] = sid[s + 1];
     }
     sid[S - 1] = -3;
@@ -477,7 +501,9 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   auto restore = [&](int p) {
     if (p >= 0 && top_id() == p) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) H[kb] = st[0][kb];
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) H[i][kb] = st[0][i][kb];
       return;
     }
     load_h0(H);  // the pool state again (rare: a later root, or a parked state dropped from the stack)
@@ -537,25 +563,36 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   }
 }
 
-template <int K, int WMAX, int S>
-int launch_k(const eagle4_records_args& a, hipStream_t s) {
-  const int tiles = e4::ceil_div(a.V, ROWS);
+template <int K, int WMAX, int S, int RT>
+int launch_rt(const eagle4_records_args& a, hipStream_t s) {
+  const int tiles = e4::ceil_div(a.V, 16 * WAVES * RT);
   const int64_t total = static_cast<int64_t>(a.N) * a.HV * tiles;
   if (total > (int64_t(1) << 30)) return EAGLE4_NOT_COVERED;
   const int per_xcd = static_cast<int>((total + 7) / 8);
   const dim3 grid(8 * per_xcd);
   if (a.state_dtype == EAGLE4_BF16)
-    gdn_replay_kernel<K, WMAX, S, e4::Bf16><<<grid, NT, 0, s>>>(a, tiles, per_xcd, static_cast<int>(total));
+    gdn_replay_kernel<K, WMAX, S, RT, e4::Bf16><<<grid, NT, 0, s>>>(a, tiles, per_xcd, static_cast<int>(total));
   else
-    gdn_replay_kernel<K, WMAX, S, e4::F16><<<grid, NT, 0, s>>>(a, tiles, per_xcd, static_cast<int>(total));
+    gdn_replay_kernel<K, WMAX, S, RT, e4::F16><<<grid, NT, 0, s>>>(a, tiles, per_xcd, static_cast<int>(total));
   return E4_LAUNCH_STATUS();
+}
+
+// Two row tiles a wave where one workgroup per head still gives each CU one, for trees of 17 to 32 nodes, whose staged
+// rows leave few workgroups per CU (K = V = 128, 48 heads, us at 1 / 2 tiles: 32 requests of 32 nodes 175 / 127, 8 of 24
+// nodes 47 / 38, but 4 of 24 nodes 26.4 / 28.2). Up to 16 nodes it changes nothing (32 requests 66 either way).
+template <int K, int WMAX, int S>
+int launch_k(const eagle4_records_args& a, hipStream_t s) {
+  if constexpr (K == 128 && WMAX == 32)
+    if (a.V % 128 == 0 && static_cast<int64_t>(a.N) * a.HV * (a.V / 128) >= 256) return launch_rt<K, WMAX, S, 2>(a, s);
+  return launch_rt<K, WMAX, S, 1>(a, s);
 }
 
 template <int K, int S>
 int launch_w(const eagle4_records_args& a, hipStream_t s) {
   if (a.width <= 16) return launch_k<K, 16, S>(a, s);
-  if constexpr (K == 256)  // the staged rows of 64 nodes would not fit LDS: up to 32
-    return a.width <= 32 ? launch_k<K, 32, S>(a, s) : EAGLE4_NOT_COVERED;
+  if (a.width <= 32) return launch_k<K, 32, S>(a, s);
+  if constexpr (K == 256)  // the staged rows of 64 nodes would not fit LDS
+    return EAGLE4_NOT_COVERED;
   else
     return launch_k<K, 64, S>(a, s);
 }
