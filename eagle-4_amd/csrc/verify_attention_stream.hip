@@ -1147,20 +1147,19 @@ __global__ __launch_bounds__(256) void verify_stream_merge(const eagle4_attn_arg
   constexpr int kGroup = 4;       // pieces in flight
   const int s = blockIdx.x;
   const int b = s / p.HR, k = s - b * p.HR;
+  // the tables in one round of loads: the request's tiles and rows, and the shares that computed the segment's first and
+  // last tiles (recorded by the stream kernel in this launch; an empty segment's entry is not written and not used)
   const int64_t* pre = reinterpret_cast<const int64_t*>(a.workspace);
-  const int64_t tiles = pre[b + 1] - pre[b];
-  if (tiles <= 0) return;
-  // the shares that computed the segment's first and last tiles (recorded by the stream kernel in this launch)
   const int32_t* const seg_w = reinterpret_cast<const int32_t*>(pre + a.num_reqs + 1) + 2 * static_cast<int64_t>(s);
+  const int64_t tiles = pre[b + 1] - pre[b];
   const int64_t w0 = seg_w[0], w1 = seg_w[1];
-  if (w0 == w1) return;  // inside one share: written directly
-  const int item = blockIdx.y * 256 + threadIdx.x;
-  const int rows_seg = p.rows_seg;
-  if (item >= rows_seg * TPR) return;
-  const int r = item / TPR, d = kCols * (item % TPR);
-  const int G = p.G, kvh = k / p.RG, rg = k - kvh * p.RG;
   const int64_t qs = e4::ld(a.query_start_loc, b);
   int64_t rows = e4::ld(a.query_start_loc, b + 1) - qs;
+  const int item = blockIdx.y * 256 + threadIdx.x;
+  const int rows_seg = p.rows_seg;
+  if (tiles <= 0 || w0 == w1 || item >= rows_seg * TPR) return;  // one share: written directly
+  const int r = item / TPR, d = kCols * (item % TPR);
+  const int G = p.G, kvh = k / p.RG, rg = k - kvh * p.RG;
   rows = rows < a.max_query_len ? rows : a.max_query_len;
   const int rho = rg * rows_seg + r;
   const int rt = rho / 16;
@@ -1213,22 +1212,21 @@ __global__ __launch_bounds__(256) void verify_stream_merge(const eagle4_attn_arg
   }
 }
 
-// The same for segments cut into many pieces (a few long requests over the whole grid): a thread takes four columns and
-// SG runs of threads share a row.
+// The same for segments cut into more pieces: a thread takes four columns, and SG runs of threads share a row.
 template <int D, int SG, typename T>
 __global__ __launch_bounds__(256) void verify_stream_merge_many(const eagle4_attn_args a, const StreamPlan p) {
   constexpr int TPR = D / 4;
   const int s = blockIdx.x;
   const int b = s / p.HR, k = s - b * p.HR;
   const int64_t* pre = reinterpret_cast<const int64_t*>(a.workspace);
-  if (pre[b + 1] - pre[b] <= 0) return;
   const int32_t* const seg_w = reinterpret_cast<const int32_t*>(pre + a.num_reqs + 1) + 2 * static_cast<int64_t>(s);
+  const int64_t tiles = pre[b + 1] - pre[b];
   const int w0 = seg_w[0], w1 = seg_w[1];
-  if (w0 == w1) return;  // inside one share: written directly
-  const int r = blockIdx.y * (256 / TPR / SG) + threadIdx.x / (TPR * SG), d = 4 * (threadIdx.x % TPR);
-  const int rows_seg = p.rows_seg, G = p.G, kvh = k / p.RG, rg = k - kvh * p.RG;
   const int64_t qs = e4::ld(a.query_start_loc, b);
   int64_t rows = e4::ld(a.query_start_loc, b + 1) - qs;
+  if (tiles <= 0 || w0 == w1) return;  // no rows, or inside one share: written directly
+  const int r = blockIdx.y * (256 / TPR / SG) + threadIdx.x / (TPR * SG), d = 4 * (threadIdx.x % TPR);
+  const int rows_seg = p.rows_seg, G = p.G, kvh = k / p.RG, rg = k - kvh * p.RG;
   rows = rows < a.max_query_len ? rows : a.max_query_len;
   const int rho = rg * rows_seg + r, t = rho / G, gq = rho - t * G;
   const bool ok = r < rows_seg && rho / 16 < p.row_tiles && t < rows;
@@ -1261,20 +1259,22 @@ int resident_groups() {
 template <int D, int C, typename T, bool FP8>
 int launch(const eagle4_attn_args& a, const StreamPlan& p, hipStream_t s) {
   verify_stream_kernel<D, C, T, FP8><<<p.nwg, 64 * (C + kProducers), 0, s>>>(a, p);
-  // Segments of many pieces (shares per segment, on average) fold them in parallel; from five on that is faster if the rows
-  // leave room for more runs (1 request of 16384 keys, 4 KV heads at D 128: 129 pieces 35 -> 6.3 us; 4 of 2048 keys 8.5 ->
-  // 5.5 us; 16 of 1024 keys at D 64, 9 pieces 6.2 -> 4.4 us).
+  // Segments of more than two pieces (shares per segment, on average) are folded four columns a thread, eight pieces in
+  // flight (24 / 4 heads of D 256: 16 requests of 512 - 4096 keys 13.3 -> 9.5 us, 32 of 1024 - 4096 14.2 -> 11.2; 64 of
+  // 1024 - 8192, two pieces, 16.4 us by verify_stream_merge, 17.2 so), from five pieces on by parallel runs where the
+  // rows leave room for them (1 of 16384 keys, 4 KV heads at D 128, 129 pieces 35 -> 6.3 us; 4 of 2048 8.5 -> 5.5 us; 16
+  // of 1024 at D 64, 9 pieces 6.2 -> 4.4 us).
   const int64_t segs = static_cast<int64_t>(a.num_reqs) * p.HR, pieces = p.nwg / segs + 1;
-  constexpr int kMergeThreadsPerRow = D / (D < 16 ? D : 16);
-  return with_merge_runs<D>(pieces > 4 ? pieces + kMergeGroup : 1, segs * p.rows_seg, [&](auto runs) {
-    constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
-    if constexpr (SG > 1)
+  if (pieces > 2)
+    return with_merge_runs<D>(pieces > 4 ? pieces + kMergeGroup : 1, segs * p.rows_seg, [&](auto runs) {
+      constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
       verify_stream_merge_many<D, SG, T><<<dim3(segs, e4::ceil_div(p.rows_seg, RPB)), 256, 0, s>>>(a, p);
-    else
-      verify_stream_merge<D, T><<<dim3(segs, e4::ceil_div(static_cast<int64_t>(p.rows_seg) * kMergeThreadsPerRow, 256)),
-                                  256, 0, s>>>(a, p);
-    return E4_LAUNCH_STATUS();
-  });
+      return E4_LAUNCH_STATUS();
+    });
+  constexpr int kMergeThreadsPerRow = D / (D < 16 ? D : 16);
+  verify_stream_merge<D, T><<<dim3(segs, e4::ceil_div(static_cast<int64_t>(p.rows_seg) * kMergeThreadsPerRow, 256)), 256,
+                              0, s>>>(a, p);
+  return E4_LAUNCH_STATUS();
 }
 
 // The instantiations: head dims 32 .. 256, 2 / 4 / 6 consumer waves (a group of row tiles takes the smallest that
