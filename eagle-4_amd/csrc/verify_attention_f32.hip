@@ -104,6 +104,25 @@ __global__ __launch_bounds__(64 * kTilesF) void verify_f32_kernel(const eagle4_a
   const float* vn = static_cast<const float*>(a.v_new) + rq.start * a.stride_vnt + kvh * a.stride_vnh;
   const int32_t* bt = static_cast<const int32_t*>(a.block_table.ptr) + b * a.block_table.s0;
 
+  // The pages of a tile's rows are looked up a tile ahead of its loads: looked up where they were used, every tile's loads
+  // (and the products after them) waited for the page table first (kernel and merge, 16 / 4 heads of D 128: 2 requests of
+  // 2048 keys 43 -> 28 us, 1 of 512 20 -> 16.5; D 64, 4 of 2048 32 -> 18; D 256, 16 of 4096 915 -> 749, now bound by
+  // the fp32 products).
+  const int page_shift = (a.page & (a.page - 1)) == 0 ? __builtin_ctz(a.page) : -1;
+  auto key_at = [&](int tile, int kk) {  // keys past the split: its last one, masked later
+    const int p0 = lo + tile * kKeysF + kk;
+    return p0 < hi ? p0 : hi - 1;
+  };
+  auto page_at = [&](int pos) { return page_shift >= 0 ? pos >> page_shift : pos / a.page; };
+  int32_t pages[TL::PER];
+  auto lookup = [&](int tile) {
+    if (tile >= n_ctx) return;
+#pragma unroll
+    for (int i = 0; i < TL::PER; ++i) {
+      const int e = tid + 256 * i;
+      pages[i] = bt[page_at(key_at(tile, (e < TL::Q4 ? e : 0) / (D / 4)))];
+    }
+  };
   // a tile's K / V rows into registers: float4 e = tid + 256 i is key e / (D / 4), d 4 (e % (D / 4)); keys past the
   // split (or the draft rows) read the last valid one, masked later
   f32x4_t rk[TL::PER], rv[TL::PER];  // native vectors: an array of them stays in registers
@@ -121,10 +140,9 @@ __global__ __launch_bounds__(64 * kTilesF) void verify_f32_kernel(const eagle4_a
           ks = kn + j * a.stride_knt;
           vs = vn + j * a.stride_vnt;
         } else {
-          const int p0 = lo + tile * kKeysF + kk;
-          const int pos = p0 < hi ? p0 : hi - 1;
-          const int64_t blk = bt[pos / a.page];
-          const int64_t sl = pos % a.page;
+          const int pos = key_at(tile, kk);
+          const int64_t blk = pages[i];
+          const int64_t sl = pos - page_at(pos) * a.page;
           ks = kc + blk * a.stride_kb + sl * a.stride_ks;
           vs = vc + blk * a.stride_vb + sl * a.stride_vs;
         }
@@ -153,12 +171,15 @@ __global__ __launch_bounds__(64 * kTilesF) void verify_f32_kernel(const eagle4_a
   for (int i = 0; i < D / 16; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
+  lookup(0);
   if (n_tiles > 0) load(0);
+  lookup(1);
   for (int tile = 0; tile < n_tiles; ++tile) {
     __syncthreads();  // the previous tile is no longer read
     stage();
     __syncthreads();
     if (tile + 1 < n_tiles) load(tile + 1);
+    lookup(tile + 2);
     const bool is_new = tile >= n_ctx;
     const int base = is_new ? (tile - n_ctx) * kKeysF : lo + tile * kKeysF;
 
