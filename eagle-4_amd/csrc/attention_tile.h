@@ -242,7 +242,6 @@ constexpr int kStreamMaxReqs = 1024;  // per-request query starts and contexts a
 
 struct StreamPlan {
   int G, row_tiles, C, RG, HR, rows_seg, nwg, direct, fp8;
-  int cus;
   int seg_cost;  // a segment's end in quarter tiles, for the cost-weighted shares
   int64_t part_off, lse_off;  // float offsets into the workspace (the int64 prefix of tiles per request is first)
 };
@@ -324,29 +323,14 @@ int with_merge_runs(int64_t partials, int64_t rows, F&& go) {
   return go(std::integral_constant<int, 1>{});
 }
 
-// The keys per split of a call that the split schedule serves better than the streamed one, 0 for the others. A small job
-// is bound by the streamed schedule's per-workgroup setup (~10 us of table loads, share search and ring fill before the
-// first tile) and, with several requests, its segment ends; the split schedule has neither, as long as one round of
-// workgroups (one per CU at D 256, two below) takes the whole block tables and the splits stay short enough for the
-// balance not to matter. The shortest splits that fit one round, from 96 keys up (32 and 64 keys are no faster: 1 request
-// of 512 keys 16.3 and 13.9 against 14.0 us). Measured with the merge, streamed / split, 16-bit pages: 16 / 4 heads of
-// D 128: 2 requests of 1024 keys 20.1 / 14.4, 8 of 512 21.9 / 16.5, 16 of 1024 32.7 / 28.1, 32 of 512 34.6 / 27.6, 8 of
-// 4096 38.9 / 36.6, but 32 of 1024 - 2048 47.8 / 52.0; 24 / 4 heads of D 256: 2 of 1024 28.0 / 22.1, but 4 of 2048
-// 30.3 / 32.2; 8 / 2 heads of D 64: 4 of 2048 19.2 / 12.5, 32 of 512 20.3 / 15.8, but 32 of 2048 24.0 / 26.2. fp8 pages
-// (whose scales the streamed schedule applies in fp32, the split one to the 16-bit keys) keep to one request of up to
-// 4096 keys. A caller's own chunk is kept.
-inline int small_job_chunk(const eagle4_attn_args& a) {
-  const int64_t capacity = static_cast<int64_t>(a.max_blocks) * a.page;
-  if (a.chunk > 0) return 0;
-  if (a.cache_dtype == EAGLE4_FP8_E4M3) return a.num_reqs == 1 && capacity <= 4096 ? 96 : 0;
-  const int most = a.D == 256 ? 96 : a.D == 128 ? 256 : 192, round = a.D == 256 ? 256 : 512;
-  const int64_t row_groups = e4::ceil_div(e4::ceil_div(static_cast<int64_t>(a.Hq / a.Hkv) * a.max_query_len, 16), 8);
-  const int64_t columns = static_cast<int64_t>(a.num_reqs) * a.Hkv * row_groups;
-  if (capacity > int64_t(round) * most) return 0;
-  for (int chunk = 96; chunk <= most; chunk += kTileKeys)
-    if (columns * e4::ceil_div(capacity, chunk) <= round) return chunk;
-  return 0;
+// One request whose block table holds at most 4096 keys is too small for the streamed schedule's per-workgroup setup
+// (~10 us of table loads, share search and ring fill before the first tile): the split schedule with 96-key splits
+// finishes sooner (batch 1, L 512, D 128 bf16: 15.5 against 18.4 us; splits of 32 / 64 keys 19.3 / 16.3 us). A
+// caller's own chunk is kept.
+inline bool small_attention_job(const eagle4_attn_args& a) {
+  return a.chunk <= 0 && a.num_reqs == 1 && static_cast<int64_t>(a.max_blocks) * a.page <= 4096;
 }
+constexpr int kSmallJobChunk = 96;
 
 bool stream_covered(const eagle4_attn_args& a);
 bool stream_plan(const eagle4_attn_args& a, StreamPlan& p);

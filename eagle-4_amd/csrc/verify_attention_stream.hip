@@ -113,18 +113,9 @@ E4_DEV int tiles_of(const int* s_qsl, const int* s_ctx, int b) {
   return (s_ctx[b] + CK - 1) / CK + (wk + kTileKeys - 1) / kTileKeys;
 }
 
-// The shares that take work: at least kMinTilesPerGroup tiles each. fp8 tiles hold twice the keys and take a consumer
-// 2.5 times a 16-bit tile's time, so half as many while that keeps to one share per CU (24 / 4 heads of D 256: 2 requests
-// of 1024 keys 41.2 -> 30.6 us, 16 of 1024 49.8 -> 38.1 us; past one per CU two share one: 1 of 16384, 16 / 4 heads of
-// D 128, 257 shares 34.7 against 28.2 us). 16-bit tiles gain nothing, and their weighted shares need the longer span.
-E4_DEV int64_t active_groups(int64_t tiles_all, const StreamPlan& p) {
-  int64_t n = (tiles_all + kMinTilesPerGroup - 1) / kMinTilesPerGroup;
-  if (p.fp8) {
-    const int64_t half = (tiles_all + kMinTilesPerGroup / 2 - 1) / (kMinTilesPerGroup / 2);
-    const int64_t more = half < p.cus ? half : p.cus;
-    n = more > n ? more : n;
-  }
-  return n < p.nwg ? n : p.nwg;
+E4_DEV int64_t active_groups(int64_t tiles_all, int nwg) {
+  const int64_t n = (tiles_all + kMinTilesPerGroup - 1) / kMinTilesPerGroup;
+  return n < nwg ? n : nwg;
 }
 
 E4_DEV int page_div(int pos, int page, int shift) {
@@ -718,7 +709,7 @@ void verify_stream_kernel(const eagle4_attn_args a, const StreamPlan p) {
   }
   const int64_t total_t = total & kTileMask;
   const int64_t tiles_all = total_t * HR;
-  const int64_t nact = active_groups(tiles_all, p);
+  const int64_t nact = active_groups(tiles_all, p.nwg);
   const int64_t E = p.seg_cost;
   const int64_t cost_all = HR * (4 * total_t + E * (total >> kCnt));
   const int w = blockIdx.x;
@@ -1242,7 +1233,6 @@ __global__ __launch_bounds__(256) void verify_stream_merge_many(const eagle4_att
   *reinterpret_cast<uint2*>(o) = make_uint2(T::pack(sum.x * inv, sum.y * inv), T::pack(sum.z * inv, sum.w * inv));
 }
 
-// workgroups per CU
 template <int D, int C, typename T, bool FP8>
 int resident_groups() {
   static const int per_cu = [] {
@@ -1253,7 +1243,11 @@ int resident_groups() {
       n = 0;
     return n;
   }();
-  return per_cu;
+  int dev = 0, cus = 0;
+  if (per_cu <= 0 || hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 0;
+  return per_cu * cus;
 }
 
 template <int D, int C, typename T, bool FP8>
@@ -1324,7 +1318,7 @@ bool stream_covered(const eagle4_attn_args& a) {
                         a.D) * 2;
   const bool rows_ok = a.stride_ot >= 0 && a.stride_oh >= 0 && span < (int64_t(1) << 30);
   return (a.cache_dtype == a.dtype || fp8) && rows_ok && a.num_reqs <= kStreamMaxReqs && a.chunk <= 0 &&
-         small_job_chunk(a) == 0;
+         !small_attention_job(a);
 }
 
 bool stream_plan(const eagle4_attn_args& a, StreamPlan& p) {
@@ -1350,11 +1344,7 @@ bool stream_plan(const eagle4_attn_args& a, StreamPlan& p) {
     using K = decltype(cfg);
     return resident_groups<K::D, K::C, typename K::T, K::FP8>();
   });
-  int dev = 0;
-  if (p.nwg <= 0 || hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&p.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || p.cus <= 0)
-    return false;
-  p.nwg *= p.cus;
+  if (p.nwg <= 0) return false;
   const int64_t slots = 2 * static_cast<int64_t>(p.nwg);  // a share's first and last piece
   const int64_t rows_seg = p.rows_seg;
   // a segment's end, in quarter tiles: its rows' query loads and output stores (96 rows at D 256: 4.5 tiles' time,

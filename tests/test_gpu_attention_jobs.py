@@ -1,6 +1,6 @@
-"""Verify attention on both sides of the small-job rule (the split schedule's one round of workgroups) and of the streamed
-schedule's fp8 shares: ragged contexts (empty ones among them) against the oracle, and the split that the rule chooses
-against the same call with that split given. 2e-2 abs / 1e-2 rel, as the schedules' other tests."""
+"""Verify attention of small jobs, one request (whose short tables take the split schedule) to a few: ragged contexts (empty
+ones among them) against the oracle, and several requests under wider block tables, whose results keep their bits. 2e-2
+abs / 1e-2 rel, as the schedules' other tests."""
 
 import pytest
 import torch
@@ -34,10 +34,7 @@ def test_small_jobs(dev, batch, lmax, hq, hkv, d, page, fp8):
     torch.testing.assert_close(got.cpu().float(), want.float(), atol=2e-2, rtol=1e-2)
     no_alloc = run(verify_attention, g, torch.zeros_like(g["q"]), no_alloc=True, **on_dev)
     assert torch.equal(no_alloc, got)
-    capacity = g["block_table"].shape[1] * page
-    rows = -(-(-(-hq // hkv * 9 // 16)) // 8)
-    limit, most = (256, 96) if d == 256 else (512, 256 if d == 128 else 192)
-    chunk = next((c for c in range(96, most + 1, 32) if batch * hkv * rows * -(-capacity // c) <= limit), 0)
-    if chunk and not fp8:
-        given = run(verify_attention, g, torch.zeros_like(g["q"]), chunk=chunk)
-        assert torch.equal(given, got)
+    if batch > 1:  # the table an engine hands over is as wide as its longest allowed context: nothing follows from its width
+        table = g["block_table"]
+        g["block_table"] = torch.cat([table, table[:, :1].expand(-1, 3 * table.shape[1] + 5)], 1)
+        assert torch.equal(run(verify_attention, g, torch.zeros_like(g["q"]), **on_dev), got)
