@@ -423,11 +423,20 @@ int launch_k(const eagle4_records_args& a, hipStream_t s) {
 // column tiles) and, with few requests, by their dependence; the walk that it replaces steps through the nodes one by
 // one, each a chain of two lane sums. K = V = 128, fp32 pool, one call among others: 1 request of 24 nodes, 16 heads
 // 33.4 -> 9.4 us; 8 of 40 nodes, 48 heads 318 -> 31 us; 32 of 64 nodes, 48 heads 2108 -> 157 us.
+//   - A diagonal tile is solved by substitution over blocks of four nodes, each block by its own inverse
+//     (I + B)^-1 = I - B + B^2 - B^3. The product form of a whole tile's inverse (powers up to L^8) cancels where keys along
+//     a path are alike and gates near one: a chain of 40 nodes, keys 0.9 alike, beta and decay 1, has powers in the
+//     thousands, and deltas of order one were off by 1e-3; by substitution 1.5e-6 (the walk in fp32: 4e-7).
 //   - Decay ratios are exp2 of differences of root-path sums of log2 decays; the sums are fp64, so what two nodes share
 //     cancels exactly and the ratio's error is that of the path between them, whatever the root path's length.
 //   - A value that is not finite stays on its node and the node's descendants, as in a walk: products with zeros would
 //     spread it over the tile, so it is taken out of the right-hand sides (and a node with such a key or gate out of
 //     the products), remembered per column, and put back as NaN where the outputs of that path are stored.
+// The node at position p of the wide form's 16-row tiles (and the position of a node: its own inverse): rows 4 g + b of
+// a tile, element b of the lanes, hold nodes 4 b + g, so that what one MFMA contracts over (element b of the four lane
+// groups) is a block of four consecutive nodes.
+E4_DEV int place(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
+
 template <int K, int NTL, int NTILE, typename Tpool>
 __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records_args a, int slices, int per_xcd,
                                                              int total) {
@@ -460,18 +469,22 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
 
   // ---- every load before the first wait; rows past the tree read its last row (masked below) ------------------------
   const int par_raw = entry(a.parent, n, lane < T ? lane : T - 1);
+  const int node = place(lane);  // the node at position `lane`
   uint4 qr[NTILE][KB], kr[NTILE][KB];
   Run16<NTL> vr[NTILE][4];
   Word ga, gb;
   const int v0 = slice * 16 * NTL;
-  auto load_rows = [&](auto&& row_of) {  // row_of(position): the request's row there
-    const int64_t tl = bos + row_of(lane < T ? lane : T - 1);
+  auto load_rows = [&](auto&& row_of) {  // row_of(position): the request's row there, or one past the tree
+    auto row_at = [&](int p) {
+      const int row = row_of(p);
+      return bos + (row < T ? row : T - 1);
+    };
+    const int64_t tl = row_at(lane);
     ga = word_of(a.a, tl * a.stride_a + hv, a.gate_dtype);
     gb = word_of(a.b, tl * a.stride_b + hv, a.gate_dtype);
 #pragma unroll
     for (int I = 0; I < NTILE; ++I) {
-      const int p = 16 * I + c;
-      const int64_t tok = bos + row_of(p < T ? p : T - 1);
+      const int64_t tok = row_at(16 * I + c);
       const uint16_t* qp = static_cast<const uint16_t*>(a.q) + tok * a.stride_q + ih * K + 8 * g;
       const uint16_t* kp = static_cast<const uint16_t*>(a.k) + tok * a.stride_k + ih * K + 8 * g;
 #pragma unroll
@@ -481,13 +494,12 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = 16 * I + 4 * g + r;
-        const int64_t ti = bos + row_of(i < T ? i : T - 1);
+        const int64_t ti = row_at(16 * I + 4 * g + r);
         vr[I][r].load(static_cast<const uint16_t*>(a.v) + ti * a.stride_v + static_cast<int64_t>(hv) * a.V + v0 + NTL * c);
       }
     }
   };
-  load_rows([](int p) { return p; });
+  load_rows(place);
   using PS = typename Tpool::storage;
   constexpr int kSliceBytes = 16 * NTL * K * static_cast<int>(sizeof(PS));
   const char* slot = static_cast<const char*>(a.state) +
@@ -508,29 +520,33 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the order of the nodes: parents first -------------------------------------------------------------------------
-  // lane p is the node at position p; a parent outside the tree (or the node itself) makes the node a root
-  int par = lane > 0 && lane < T && par_raw >= 0 && par_raw < T && par_raw != lane ? par_raw : -1;
-  const bool reordered = __ballot(par > lane) != 0;
-  s_id[lane] = lane;
+  // lane r is row r here; a parent outside the tree (or the node itself) makes the node a root
+  const int par_row = lane > 0 && lane < T && par_raw >= 0 && par_raw < T && par_raw != lane ? par_raw : -1;
+  const bool reordered = __ballot(par_row > lane) != 0;
+  int rank = lane;
   if (reordered) {  // rank the rows by (depth, row)
     int depth = 0;
-    for (int it = 0, x = par; it < T; ++it) {  // one step up for every lane; all lanes take part in the shuffle
-      const int up = __shfl(par, x >= 0 ? x : 0);
+    for (int it = 0, x = par_row; it < T; ++it) {  // one step up for every lane; all lanes take part in the shuffle
+      const int up = __shfl(par_row, x >= 0 ? x : 0);
       if (x >= 0) {
         ++depth;
         x = up;
       }
     }
     const int key = lane < T ? depth * 64 + lane : 64 * 128 + lane;
-    int rank = 0;
+    rank = 0;
     for (int j = 0; j < 64; ++j) rank += readlane(key, j) < key ? 1 : 0;
-    s_id[rank] = lane;
-    __syncthreads();
-    const int parent_rank = __shfl(rank, par >= 0 ? par : 0);
-    const int by_row = par >= 0 ? parent_rank : -1;
-    par = __shfl(by_row, s_id[lane]);
-    load_rows([&](int p) { return s_id[p]; });
   }
+  s_id[place(rank)] = lane;
+  __syncthreads();
+  // from here on lane p is the node at position p
+  int par;
+  {
+    const int up = __shfl(par_row, s_id[lane]);
+    const int up_rank = __shfl(rank, up >= 0 ? up : 0);
+    par = up >= 0 ? place(up_rank) : -1;
+  }
+  if (reordered) load_rows([&](int p) { return s_id[p]; });
 
   // ---- per node (lane p): gates, ancestors, root-path log decay; squared norms from the tiles' diagonals --------------
   const float A = -expf(widen_word(A_w, a.A_log_dtype));
@@ -555,7 +571,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   const float gl = A * (x_dt <= 20.0f ? logf(1.0f + expf(x_dt)) : x_dt);  // gate_of's log decay
   uint64_t anc = par >= 0 ? 1ull << par : 0ull;
   int jmp = par;
-  double lsum = lane < T ? fmax(static_cast<double>(gl) * 1.4426950408889634, -1048576.0) : 0.0;
+  double lsum = node < T ? fmax(static_cast<double>(gl) * 1.4426950408889634, -1048576.0) : 0.0;
 #pragma unroll
   for (int it = 0; it < ROUNDS; ++it) {
     const int src = jmp >= 0 ? jmp : lane;
@@ -573,8 +589,8 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   const float2 nrm = s_nrm[lane < NN ? lane : 0];
   const float ks_l = 1.0f / sqrtf(nrm.x + 1e-6f);
   const bool finite = fabsf(nrm.x) <= 3.4e38f && fabsf(gt.x) <= 3.4e38f && fabsf(gt.y) <= 3.4e38f;
-  const uint64_t bad = __ballot(lane < T && !finite);  // nodes whose key or gate is not finite
-  const bool use = lane < T && finite;
+  const uint64_t bad = __ballot(node < T && !finite);  // nodes whose key or gate is not finite
+  const bool use = node < T && finite;
   s_nd[lane] = make_float4(use ? ks_l : 0.f, a.scale / sqrtf(nrm.y + 1e-6f), use ? gt.y : 0.f,
                            __builtin_amdgcn_exp2f(static_cast<float>(lsum)));
   s_lg[lane] = lsum;
@@ -586,7 +602,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
 #pragma unroll
     for (int I = 0; I < NTILE; ++I) {
       const int p = 16 * I + c;
-      if (p < T) {
+      if (place(p) < T) {
         float* d0 = rec + (static_cast<int64_t>(s_id[p]) * a.HV + hv) * a.rec + a.V;
         const float ks = 1.0f / sqrtf(s_nrm[p].x + 1e-6f);
 #pragma unroll
@@ -598,7 +614,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
         }
       }
     }
-    if (lane < T) rec[(static_cast<int64_t>(s_id[lane]) * a.HV + hv) * a.rec + a.V + K] = gt.x;
+    if (node < T) rec[(static_cast<int64_t>(s_id[lane]) * a.HV + hv) * a.rec + a.V + K] = gt.x;
   }
   if (bad != 0) {
 #pragma unroll
@@ -674,7 +690,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
         out[u] = mm(WT, D[J][u], out[u]);
       }
     }
-    f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, KQ = {0.f, 0.f, 0.f, 0.f}, L, LT, WT, E;
+    f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, KQ = {0.f, 0.f, 0.f, 0.f}, B, BT, LoT, WT;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       KK = mma_bf16(kr[I][kb], kr[I][kb], KK);
@@ -688,49 +704,55 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
       const double lg_i = s_lg[ni];
       const bool c_above_i = (s_anc[ni] >> (16 * I + c)) & 1, i_above_c = (anc_c >> ni) & 1;
       const float kk_n = nd[r].x * ci.x * KK[r];
-      L[r] = c_above_i ? nd[r].z * __builtin_amdgcn_exp2f(static_cast<float>(lg_i - lg_c)) * kk_n : 0.f;
       const float ratio = i_above_c || i == c ? __builtin_amdgcn_exp2f(static_cast<float>(lg_c - lg_i)) : 0.f;
-      LT[r] = i_above_c ? ci.z * ratio * kk_n : 0.f;
+      const float l = c_above_i ? nd[r].z * __builtin_amdgcn_exp2f(static_cast<float>(lg_i - lg_c)) * kk_n : 0.f;
+      const float lt = i_above_c ? ci.z * ratio * kk_n : 0.f;
+      const bool own = (c & 3) == r;  // nodes i and c in one block of four
+      B[r] = own ? l : 0.f;
+      BT[r] = own ? lt : 0.f;
+      LoT[r] = own ? 0.f : lt;
       WT[r] = i_above_c || i == c ? ratio * (ci.y * nd[r].x * KQ[r]) : 0.f;
-      E[r] = i == c ? 1.f : 0.f;
     }
-    const f32x4_t P2 = mm(LT, L), P2T = mm(L, LT);
-    const f32x4_t P4 = mm(P2T, P2), P4T = mm(P2, P2T);
-    const f32x4_t P8 = mm(P4T, P4);
-    f32x4_t TinvT = mm(E + P2, E - LT);
-    TinvT = mm(E + P4, TinvT);
-    TinvT = mm(E + P8, TinvT);
+    // (I + B)^-1 - I = B^2 - B - B B^2 for the 4 x 4 blocks B on L_II's diagonal (B^4 = 0), transposed
+    const f32x4_t B2T = mm(B, BT);
+    const f32x4_t invT = mm(B, -B2T, B2T - BT);
 #pragma unroll
     for (int u = 0; u < NTL; ++u) {
       f32x4_t rhs;
       bool off = false;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        rhs[r] = 16 * I + 4 * g + r < T
-                     ? nd[r].z * (vr[I][r].at(u) - nd[r].w * (nd[r].x * KS[I][u][r])) - sub[u][r] : 0.f;
-        off |= !(fabsf(rhs[r]) <= 3.4e38f);
+        rhs[r] = 16 * I + 4 * r + g < T ? nd[r].z * (vr[I][r].at(u) - nd[r].w * (nd[r].x * KS[I][u][r])) : 0.f;
+        off |= !(fabsf(rhs[r] - sub[u][r]) <= 3.4e38f);
       }
       if (__ballot(off) != 0) {  // take what is not finite out of the products, remember where it was
         uint32_t m = 0;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (!(fabsf(rhs[r]) <= 3.4e38f)) {
+          if (!(fabsf(rhs[r] - sub[u][r]) <= 3.4e38f)) {
             m |= 1u << (4 * g + r);
-            rhs[r] = 0.f;
+            rhs[r] = sub[u][r] = 0.f;
           }
         m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16));
         m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32));
         lost[u] |= static_cast<uint64_t>(m) << (16 * I);
         any_lost = true;
       }
-      D[I][u] = mm(TinvT, rhs);
+      // element b of the lanes is block b: its right-hand side less what the blocks before it give, then its inverse
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const float x = rhs[b] - sub[u][b];
+        const f32x4_t z = __builtin_amdgcn_mfma_f32_16x16x4f32(invT[b], x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        D[I][u][b] = x + z[b];
+        if (b < 3) sub[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(LoT[b], D[I][u][b], sub[u], 0, 0, 0);
+      }
       out[u] = mm(WT, D[I][u], out[u]);
     }
     // ---- the tile's outputs and deltas ----
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int p = 16 * I + 4 * g + r;
-      if (p >= T) continue;
+      if (place(p) >= T) continue;
       float o[NTL], d[NTL];
 #pragma unroll
       for (int u = 0; u < NTL; ++u) {
