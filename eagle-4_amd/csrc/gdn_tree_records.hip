@@ -410,10 +410,11 @@ int launch_records(const eagle4_records_args& a, hipStream_t s) {
 // One workgroup folds RPT x 4 x (64 / C) V rows of one (request x value head, layer): 4 waves, C lanes per row, a lane
 // holding 16-byte chunks of its rows (an 8-byte one at the smallest K). HBM-bound: the pool state once each way. What
 // kept it from that was a chain of round trips per workgroup, the path's parents one by one and then each node's record
-// as it was folded; now there are three: the tables with the parents (a lane per node), then the state with the records
-// of up to NST path nodes (staged in LDS, shared by all rows), then the store. 16 requests, 12 layers of 48 heads,
-// K = V = 128, bf16 pool: 188 -> 112 us, 5.8 TB/s (122 with regular stores: the states' next reader comes a forward
-// pass later, so they are loaded and stored nontemporally).
+// as it was folded; now there are four: the tables, then the request's parents (a lane per node) with the state behind
+// them, then the records of up to NST path nodes (staged in LDS, shared by all rows), then the store. 16 requests, 12
+// layers of 48 heads, K = V = 128, bf16 pool: 188 -> 111 us, 5.8 TB/s (121 with regular stores: the states' next reader
+// comes a forward pass later, so they are loaded and stored nontemporally; 109 with the parents read along with the
+// tables, which would read a row of them for requests that are skipped and need not have one).
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 typedef uint32_t u32x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
@@ -443,8 +444,10 @@ __global__ __launch_bounds__(256) void gdn_records_commit_kernel(const eagle4_re
 
   const int64_t step = uni64(e4::ld(a.commit_steps, n)), slot = uni64(e4::ld(a.state_indices, n)),
                 rrow = uni64(e4::ld(a.record_indices, n));
-  const int up = static_cast<int>(e4::ld(a.parent, n, lane < a.dmax ? lane : 0));
   if (!(step >= 0 && slot >= 0 && rrow >= 0)) return;
+  // Behind the test: a skipped request (a batch padded with -1) need not have a row of parents, nor one at its root.
+  int up = -1;
+  if (step > 0 && step < a.dmax) up = static_cast<int>(e4::ld(a.parent, n, lane < a.dmax ? lane : 0));
 
   // the state, in flight while the path and its records are looked up
   PS* st[RPT];

@@ -41,3 +41,29 @@ def test_commit_tilings(dev, dims, layers, n, pool_dtype, spare, width):
         torch.testing.assert_close(got.cpu().float(), want.float(), atol=1e-2, rtol=1e-2)
     else:
         assert_states_close(got.cpu(), want)
+
+
+@pytest.mark.parametrize("pool_dtype", [torch.bfloat16, torch.float32])
+def test_skipped_requests_have_no_parents(dev, pool_dtype):
+    """A batch padded past its parent table's rows: the padding is skipped (a negative step, slot or row) or accepted at
+    its root, which has no parent, and none of that reads the table."""
+    from eagle_harness.kernels.gdn_tree_records import gdn_tree_records_commit
+
+    announce(f"records commit, padded batch {pool_dtype}")
+    gen = torch.Generator().manual_seed(3)
+    layers, n, width, HV, V, K = 2, 6, 9, 2, 64, 128
+    parent = torch.tensor([[-1, 0, 1, 2, 3, 4, 5, 6, 7], [-1, 0, 0, 1, 1, 2, 2, 3, 3]])
+    state = (torch.randn(layers, n + 1, HV, V, K, generator=gen) * 0.1).to(pool_dtype)
+    records = torch.randn(layers, n, width, HV, V + K + 1, generator=gen) * 0.1
+    slots, rows = torch.tensor([1, 2, 3, -1, 5, 6]), torch.tensor([0, 1, 2, 3, -1, 5])
+    steps = torch.tensor([8, 7, -1, 4, 4, 0])
+    rounded = pool_dtype != torch.float32
+    want = state.clone()
+    orec.gdn_tree_records_commit(want, records, slots, rows, steps, parent, rounded)
+    got = state.to(dev)
+    gdn_tree_records_commit(got, records.to(dev), slots.to(dev), rows.to(dev), steps.to(dev), parent.to(dev), rounded)
+    if rounded:
+        torch.testing.assert_close(got.cpu().float(), want.float(), atol=1e-2, rtol=1e-2)
+    else:
+        assert_states_close(got.cpu(), want)
+    assert torch.equal(got.cpu()[:, [0, 3, 4, 5]], state[:, [0, 3, 4, 5]])
