@@ -186,10 +186,12 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_tree_walk_kernel(const eagle4_
   const int plan = ps.plan[lane];  // read before the walk writes s_out (after the next barrier)
   const bool dfs = ps.dfs != 0;
   // L2 norms over K (:143-151) and q^, k^ (read by every node of the walk) in one pass
-  if (STAGED > 16 && ts <= TS / 2)  // twice the threads a node
-    stage_norms<Tin, K, TS, NT, TS / 2>(s_qr, s_kr, s_sc, ts, tid, a.scale, s_q, s_k);
-  else
+  if constexpr (STAGED > 16) {  // with the sums of the 16-node form: its staged nodes, then those that it would load itself
+    stage_norms<Tin, K, TS, NT, TS / 2>(s_qr, s_kr, s_sc, ts < TS / 2 ? ts : TS / 2, tid, a.scale, s_q, s_k);
+    if (ts > TS / 2) stage_norms_lanes<Tin, K, C, TS, NT>(s_qr, s_kr, s_sc, TS / 2, ts, tid, a.scale, s_q, s_k);
+  } else {
     stage_norms<Tin, K, TS, NT>(s_qr, s_kr, s_sc, ts, tid, a.scale, s_q, s_k);
+  }
   __syncthreads();  // the raw rows' space becomes the stack
 
   settle_loads();  // the initial state and the plan tables

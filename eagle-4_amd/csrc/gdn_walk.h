@@ -292,4 +292,41 @@ E4_DEV void stage_norms(const typename Tin::storage (&s_q)[TS][K], const typenam
   }
 }
 
+// The same for the staged nodes from `first` on in a walk's own lane layout, C lanes a node, each the 16-byte chunks
+// 4 C j + 4 c: the order in which the walk sums a node that it loads itself, so a node's bits do not depend on whether it
+// is staged.
+template <typename Tin, int K, int C, int TS, int NT>
+E4_DEV void stage_norms_lanes(const typename Tin::storage (&s_q)[TS][K], const typename Tin::storage (&s_k)[TS][K],
+                              float4 (&s_sc)[TS], int first, int ts, int tid, float scale, float (&qh)[TS][K],
+                              float (&kh)[TS][K]) {
+  constexpr int E = K / C;
+  static_assert(NT / C >= TS / 2, "a node per C threads, half of the staged ones at once");
+  const int t = first + tid / C, c = tid % C;
+  float qq = 0.f, kk = 0.f;
+  float qv[E], kv[E];
+  if (t < ts) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int at = 4 * C * (e / 4) + 4 * c + e % 4;
+      qv[e] = Tin::to_f32(s_q[t][at]);
+      kv[e] = Tin::to_f32(s_k[t][at]);
+      qq = fmaf(qv[e], qv[e], qq);
+      kk = fmaf(kv[e], kv[e], kk);
+    }
+  }
+  const float qs = scale / sqrtf(e4::group_sum<C>(qq) + 1e-6f), ks = 1.0f / sqrtf(e4::group_sum<C>(kk) + 1e-6f);
+  if (t < ts) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int at = 4 * C * (e / 4) + 4 * c + e % 4;
+      qh[t][at] = qv[e] * qs;
+      kh[t][at] = kv[e] * ks;
+    }
+    if (c == 0) {
+      s_sc[t].z = qs;
+      s_sc[t].w = ks;
+    }
+  }
+}
+
 }  // namespace e4walk
