@@ -340,7 +340,8 @@ __global__ __launch_bounds__(NT) void gdn_replay_kernel(const eagle4_records_arg
   // per node: |q|^2, |k|^2 and k . q over K (:147-150), LPN0 adjacent threads a node, the first LPN of them each
   // summing a contiguous run
   {
-    constexpr int LPN0 = NT / WMAX;
+    // 32 staged rows of K <= 128 sum as 64 do (four threads a node): a tree's bits do not depend on how many are staged
+    constexpr int LPN0 = NT / (WMAX == 32 && K < 256 ? 64 : WMAX);
     constexpr int LPN = LPN0 < K / 4 ? LPN0 : K / 4;
     constexpr int PER = K / LPN;
     static_assert(PER % 4 == 0 && LPN0 <= 16, "norm split");

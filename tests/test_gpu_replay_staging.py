@@ -37,3 +37,22 @@ def test_replay_stagings(dev, width, n, dims, dtype):
     got = _call(gdn_tree_records_update, g, width, tree_paths=g["tree_paths"])
     torch.cuda.synchronize()
     _compare(got, want, g["records"], want_rec, False, dims[2], dims[3])
+
+
+@pytest.mark.parametrize("n,dims,dtype", [(3, (2, 4, 128, 128), torch.bfloat16), (22, (2, 12, 128, 128), torch.float16),
+                                          (3, (1, 2, 64, 48), torch.bfloat16), (2, (1, 1, 32, 16), torch.bfloat16)])
+def test_staged_counts_agree(dev, n, dims, dtype):
+    """The same trees under tables of 32 and of 40 columns (32 and 64 staged nodes): the same outputs and records, bit for bit."""
+    from eagle_harness.kernels.gdn_tree_records import gdn_tree_records_update
+
+    announce(f"replay staged counts n={n} dims={dims} {dtype}")
+    rng = np.random.default_rng(n)
+    trees = [seeded_tree(rng, 17 + 5 * i % 16) for i in range(n)]
+    got = []
+    for width in (32, 40):
+        inp, _ = _inputs(trees, *dims, dtype, in_dtype=dtype, seed=n, width=width)
+        g = _to(inp, dev)
+        out = _call(gdn_tree_records_update, g, width, tree_paths=g["tree_paths"])
+        got.append((out, g["records"][:, :32]))
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1], got[1][1])
