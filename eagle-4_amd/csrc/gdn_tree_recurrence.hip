@@ -518,19 +518,23 @@ extern "C" int eagle4_gdn_tree_recurrent_update(const eagle4_gdn_args* a, void* 
       // jumping, then a pass per tree level): they walk children in index order and park up to four states instead
       // of two, enough for the nesting of index order in drafted trees (a parent beyond them reloads its snapshot),
       // and store their snapshots nontemporally.
-      // Trees of more than 16 rows (known here only from a per-row slot table's columns) have 32 nodes staged instead of
-      // 16: a node past the staged ones is loaded in the walk, where its loads wait for every snapshot store in flight. On
-      // the small grids always (1 request of 32 nodes, 32 heads, fp32 53.7 -> 29.6 us; 16 nodes under a 32-column table
-      // 19.5 us both ways). The larger ones pay with a third of their workgroups per CU, so there from the widths on
-      // where it was faster (layer, us, 16 / 32 staged: fp32 4 requests of 24 rows 64.5 / 61.6, 16 of 24 rows 175 / 174,
-      // 64 of 24 rows 654 / 684, 64 of 32 rows 941 / 928; bf16 4 of 20 rows 47 / 41, 64 of 17 rows 317 / 363, 64 of 24
-      // rows 567 / 475, 64 of 32 rows 818 / 601).
-      const int cols = a->row_slots ? a->num_slot_cols : 0;
+      // Trees of more than 16 rows have 32 nodes staged instead of 16: a node past the staged ones is loaded in the walk,
+      // where its loads wait for every snapshot store in flight. The requests' rows are on the GPU; what is known here is
+      // their mean, from the launch's tokens, and the per-row slot table's columns, which bound them (the table may be far
+      // wider than the trees: 64 requests of 16 rows under 32 columns with a bf16 pool 277 us with 16 staged, 332 with 32).
+      // On the small grids from 17 rows on (1 request of 32 nodes, 32 heads, fp32 53.7 -> 30.4 us; 16 nodes 20.3 / 21.1).
+      // The larger ones pay with a third of their workgroups per CU, so there from the mean on where it was faster, in
+      // batches of one tree size and of sizes from half the widest (layer, us, 16 / 32 staged: bf16 4 requests of 18 rows
+      // 43.5 / 40.9, 16 of 18 rows 105.8 / 105.9, of 20 rows 122 / 114, 64 of 18 rows 361 / 381, of 20 rows 428 / 410, of
+      // 14 to 28 rows 477 / 430, of 26 rows 635 / 507; fp32 4 of 18 rows 44.8 / 45.3, of 22 rows 57.8 / 52.2, 8 of 14 to 28
+      // rows 94 / 97, of 22 rows 95.9 / 94.1, 16 of 22 rows 162 / 164, of 26 rows 195 / 191, 64 of 26 rows 688 / 700, of 32
+      // rows 941 / 865).
+      const int64_t mean = a->tokens > 0 ? e4::ceil_div(static_cast<int64_t>(a->tokens), a->N) : 0;
+      const int64_t nodes = !a->row_slots ? 0 : mean < a->num_slot_cols ? mean : a->num_slot_cols;
       const bool exact = a->snap_dtype == EAGLE4_F32;
-      const bool wide = groups8 <= 256    ? cols > 16
-                        : groups8 <= 1024 ? cols >= (exact ? 24 : 20)
-                        : groups8 <= 2048 ? cols >= 24
-                                          : cols >= (exact ? 30 : 24);
+      const bool wide = groups8 <= 256 ? nodes > 16
+                        : exact        ? nodes >= (groups8 <= 1024 ? 22 : groups8 <= 2048 ? 24 : 30)
+                                       : nodes >= (groups8 <= 1024 ? 18 : 20);
       if (groups8 <= 256)
         return wide ? launch_in<128, 16, 1, 4, 4, true, 32>(*a, s) : launch_in<128, 16, 1, 4, 4, true>(*a, s);
       if (wide) return launch_in<128, 8, 1, 4, 2, false, 32>(*a, s);

@@ -122,7 +122,8 @@ class GdnArgs(ctypes.Structure):
         "A_log:p dt_bias:p A_log_dtype:i dt_bias_dtype:i softplus_beta:f softplus_threshold:f scale:f out_dtype:i "
         "out:p stride_o:q parents:t cu_seqlens:t h0_source:p stride_h0_source:q h0_dtype:i snap_dtype:i "
         "h0_indices:t num_accepted:t snap:p stride_snap_slot:q stride_snap_row:q snap_indices:t publish:p "
-        "stride_publish:q num_slot_cols:i N:i H:i HV:i K:i V:i row_slots:i skip_chain_reload:i pad_slot_id:i"
+        "stride_publish:q num_slot_cols:i N:i H:i HV:i K:i V:i row_slots:i skip_chain_reload:i pad_slot_id:i "
+        "tokens:i"
     )
 
 

@@ -220,6 +220,7 @@ def gdn_tree_recurrent_update(
         row_slots=int(row_slots),
         skip_chain_reload=int(fp32_state),
         pad_slot_id=pad_slot_id,
+        tokens=q.shape[1],
     )
     _native.launch("eagle4_gdn_tree_recurrent_update", args, q.device)
     return out

@@ -159,6 +159,7 @@ typedef struct eagle4_gdn_args {
   int32_t row_slots;
   int32_t skip_chain_reload;
   int32_t pad_slot_id;
+  int32_t tokens; /* rows of q, over all requests; 0 if not known (it chooses between kernels of the same results) */
 } eagle4_gdn_args;
 int eagle4_gdn_tree_recurrent_update(const eagle4_gdn_args* args, void* stream);
 
