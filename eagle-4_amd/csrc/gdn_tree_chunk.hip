@@ -431,7 +431,8 @@ int launch_k(const eagle4_records_args& a, hipStream_t s) {
 //     cancels exactly and the ratio's error is that of the path between them, whatever the root path's length.
 //   - A value that is not finite stays on its node and the node's descendants, as in a walk: products with zeros would
 //     spread it over the tile, so it is taken out of the right-hand sides (and a node with such a key or gate out of
-//     the products), remembered per column, and put back as NaN where the outputs of that path are stored.
+//     the products), remembered per column, and put back where the outputs of that path are stored: NaN, as in the walk,
+//     whose states then hold infinities of both signs; the delta of an infinite value itself stays infinite.
 // The node at position p of the wide form's 16-row tiles (and the position of a node: its own inverse): rows 4 g + b of
 // a tile, element b of the lanes, hold nodes 4 b + g, so that what one MFMA contracts over (element b of the four lane
 // groups) is a block of four consecutive nodes.
@@ -449,6 +450,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   __shared__ uint64_t s_anc[64];  // per node: strict ancestors
   __shared__ float2 s_nrm[64];    // per node: |k|^2, |q|^2
   __shared__ int s_id[64];        // position -> row of the request
+  __shared__ float s_raw[NTL][4][64];  // a tile's right-hand sides that are not finite, each lane its own
 
   const int w = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
   if (w >= total) return;
@@ -588,10 +590,12 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   __syncthreads();
   const float2 nrm = s_nrm[lane < NN ? lane : 0];
   const float ks_l = 1.0f / sqrtf(nrm.x + 1e-6f);
-  const bool finite = fabsf(nrm.x) <= 3.4e38f && fabsf(gt.x) <= 3.4e38f && fabsf(gt.y) <= 3.4e38f;
-  const uint64_t bad = __ballot(node < T && !finite);  // nodes whose key or gate is not finite
-  const bool use = node < T && finite;
-  s_nd[lane] = make_float4(use ? ks_l : 0.f, a.scale / sqrtf(nrm.y + 1e-6f), use ? gt.y : 0.f,
+  const bool gates = fabsf(gt.x) <= 3.4e38f && fabsf(gt.y) <= 3.4e38f;
+  const uint64_t inf_k = __ballot(node < T && !(nrm.x <= 3.4e38f));
+  const uint64_t inf_q = __ballot(node < T && !(nrm.y <= 3.4e38f));
+  uint64_t bad = inf_k | __ballot(node < T && !gates);  // nodes whose key or gate is not finite
+  const bool use = node < T && gates;
+  s_nd[lane] = make_float4(use && ((bad >> lane) & 1) == 0 ? ks_l : 0.f, a.scale / sqrtf(nrm.y + 1e-6f), use ? gt.y : 0.f,
                            __builtin_amdgcn_exp2f(static_cast<float>(lsum)));
   s_lg[lane] = lsum;
   s_anc[lane] = anc;
@@ -654,7 +658,21 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
   uint64_t lost[NTL];  // column v0 + NTL c + u: the nodes whose right-hand side is not finite
 #pragma unroll
   for (int u = 0; u < NTL; ++u) lost[u] = 0;
-  bool any_lost = bad != 0;
+  // A row of finite elements whose squared norm overflows is a zero row once normalised (1 / inf): the key is out of the
+  // products already, and its node is not bad. One that holds an infinity or a NaN stays what it is.
+  uint64_t zero_q = 0;
+  bool any_lost = (bad | inf_q) != 0;
+  if (any_lost) {
+    auto rows_with_inf = [&](const void* x, int64_t stride) -> uint64_t {  // read again, a lane its own row
+      const uint16_t* p = static_cast<const uint16_t*>(x) + (bos + (node < T ? s_id[lane] : 0)) * stride + ih * K;
+      bool hit = false;
+#pragma unroll 1
+      for (int e = 0; e < K; ++e) hit |= (p[e] & 0x7f80u) == 0x7f80u;
+      return __ballot(hit);
+    };
+    bad &= ~inf_k | rows_with_inf(a.k, a.stride_k) | __ballot(!use);
+    zero_q = inf_q & ~rows_with_inf(a.q, a.stride_q);
+  }
 #pragma unroll
   for (int I = 0; I < NTILE; ++I) {
     if (16 * I >= T) break;
@@ -731,6 +749,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
         for (int r = 0; r < 4; ++r)
           if (!(fabsf(rhs[r] - sub[u][r]) <= 3.4e38f)) {
             m |= 1u << (4 * g + r);
+            s_raw[u][r][lane] = rhs[r] - sub[u][r];
             rhs[r] = sub[u][r] = 0.f;
           }
         m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16));
@@ -760,10 +779,16 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
         d[u] = D[I][u][r];
       }
       if (any_lost) {
-        const uint64_t path = s_anc[p] | (1ull << p);
+        const uint64_t above = s_anc[p], self = 1ull << p;
 #pragma unroll
         for (int u = 0; u < NTL; ++u)
-          if ((path & (lost[u] | bad)) != 0) o[u] = d[u] = __builtin_nanf("");
+          if (((above | self) & (lost[u] | bad)) == 0) {
+            if ((zero_q & self) != 0) o[u] = 0.f;
+          } else {
+            o[u] = __builtin_nanf("");
+            const float own = s_raw[u][r][lane];  // an infinite value's own delta
+            d[u] = (lost[u] & self) != 0 && (above & (lost[u] | bad)) == 0 ? own : __builtin_nanf("");
+          }
       }
       const int row = s_id[p];
       const int64_t col = static_cast<int64_t>(hv) * a.V + v0 + NTL * c;

@@ -58,3 +58,53 @@ def test_values_that_are_not_finite_stay_on_their_path(dev, what):
     assert torch.equal(got[0][~hit], want[0][~hit])
     row = int(inp["record_indices"][0])
     assert torch.equal(g["records"][row, : len(tree), :, :32].isnan(), hit)
+
+
+@pytest.mark.parametrize("dims,n", [((1, 2, 128, 32), 1), ((2, 16, 64, 64), 16)])  # one and two column tiles a wave
+def test_rows_whose_norm_overflows_are_zero_rows(dev, dims, n):
+    """Finite keys and queries of magnitude 1e30: their squared norm is infinite in fp32, so they normalise to zero, as in
+    the recurrence; nothing becomes NaN."""
+    from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
+
+    announce(f"records chunk form, overflowing norms {dims}")
+    tree = [-1, 0, 1, 2, 0, 4, 5] + list(range(6, 30)) + [0, 31, 32]
+    got = []
+    for big in (True, False):
+        inp, width = _inputs([tree] * n, *dims, torch.float32, seed=4)
+        for i in range(n):
+            for what, node in (("k", 5), ("k", 20), ("q", 3), ("q", 20)):
+                row = inp[what][0, i * len(tree) + node]
+                row[:] = torch.sign(row) * 1e30 if big else 0.0
+        g = _to(inp, dev)
+        out = _call(gdn_tree_chunk_update, g, width)
+        got.append((out, g["records"]))
+    assert not got[0][0].isnan().any()
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("dims,n", [((1, 2, 128, 32), 1), ((2, 16, 64, 64), 16)])
+def test_an_infinite_value_keeps_its_own_delta(dev, dims, n):
+    """An infinite value's delta is that infinity; its node's output and everything below in that column are NaN, from
+    states that hold infinities of both signs."""
+    from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
+
+    announce(f"records chunk form, infinite value {dims}")
+    tree = [-1, 0, 1, 2, 0, 4, 5] + list(range(6, 30)) + [0, 31, 32]
+    inp, width = _inputs([tree] * n, *dims, torch.float32, seed=5)
+    for i in range(n):
+        inp["v"][0, i * len(tree) + 5, 1, 3] = -float("inf")
+        inp["v"][0, i * len(tree) + 9, 1, 3] = float("inf")  # below the first
+    g = _to(inp, dev)
+    out = _call(gdn_tree_chunk_update, g, width)
+    below = [5]
+    for j in range(6, len(tree)):
+        if tree[j] in below:
+            below.append(j)
+    hit = torch.zeros(len(tree), *out.shape[2:], dtype=torch.bool)
+    hit[below, 1, 3] = True
+    for i in range(n):
+        rec = g["records"][int(inp["record_indices"][i]), : len(tree), :, : dims[3]].cpu()
+        assert rec[5, 1, 3] == -float("inf")
+        assert torch.equal(rec.isnan(), hit & (torch.arange(len(tree)) != 5)[:, None, None])
+        assert torch.equal(out[0, i * len(tree) : (i + 1) * len(tree)].cpu().isnan(), hit)
