@@ -10,15 +10,15 @@
 // record's delta, so the records hold (D, K, exp(g)) and the commit replays them.
 //
 // One wave per (request, value head, slice of 16 NTL value columns), 16 nodes on the 16 rows of the 16x16 MFMA
-// accumulator (lane (g, c), element r: row 4 g + r, column c):
+// accumulator (lane (g, c), element r: row 4 g + r, column c), each at its place():
 //   - everything the wave reads is issued first: parents, gates, q / k rows, v, the pool slice;
 //   - K K^T, K Q^T and Q Q^T on v_mfma_f32_16x16x32_bf16 from the raw bf16 rows (products exact, fp32 sums); the
 //     squared norms are the diagonals, and the norms enter as per-row factors;
 //   - per node (lane c): decay / beta, and by pointer jumping over the parent links the ancestor set (a 16-bit mask)
 //     and the root-path log2-decay sum log2 G; the decay ratios are then hardware exp2 of log2 differences;
 //   - L, L^T and W^T masked and scaled from K K^T and K Q^T;
-//   - (I + L)^-1 = (I - L)(I + L^2)(I + L^4)(I + L^8) (L is strictly lower in the ancestor order, L^16 = 0) by 8
-//     products on v_mfma_f32_16x16x4f32, kept transposed as the left operand of D = Tinv rhs;
+//   - the triangular system by substitution over blocks of four nodes on v_mfma_f32_16x16x4f32, parents in front of
+//     their children (rows given in another order are first ranked by depth);
 //   - per 16-column tile, K S0^T and Q S0^T on the bf16 MFMA with the pool state split into exact bf16 terms
 //     (1 for a bf16 pool, 2 for fp16, 3 for fp32), then rhs, D and O on the fp32 MFMA.
 // Tile u of a wave covers the columns v0 + NTL c + u, so each lane ends with NTL adjacent columns of every row it
@@ -53,6 +53,32 @@ E4_DEV f32x4_t mm(f32x4_t xt, f32x4_t y, f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[kb], y[kb], acc, 0, 0, 0);
   return acc;
+}
+
+// The node at position p of a tile's 16 rows (and the position of a node: its own inverse): rows 4 g + b, element b of the
+// lanes, hold nodes 4 b + g, so that what one MFMA contracts over (element b of the four lane groups) is a block of four
+// consecutive nodes.
+E4_DEV int place(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
+
+// A tile's triangular system by substitution over its blocks of four nodes: the blocks' own inverses, less I and
+// transposed, (I + B)^-1 - I = B^2 - B - B^3 for the 4 x 4 blocks B of L (B^4 = 0), and with them D of (I + L) D = rhs - sub,
+// LoT the rest of L transposed: element b of the lanes is block b, its right-hand side less what the blocks before it
+// give. The product form of the whole inverse (powers up to L^8) cancels where keys along a path are alike and gates
+// near one: the powers reach the thousands, and deltas of order one were off by 1e-3, by substitution 2e-6.
+E4_DEV f32x4_t block_inverses(f32x4_t B, f32x4_t BT) {
+  const f32x4_t B2T = mm(B, BT);
+  return mm(B, -B2T, B2T - BT);
+}
+E4_DEV f32x4_t solve_tile(f32x4_t invT, f32x4_t LoT, f32x4_t rhs, f32x4_t sub) {
+  f32x4_t D;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const float x = rhs[b] - sub[b];
+    const f32x4_t z = __builtin_amdgcn_mfma_f32_16x16x4f32(invT[b], x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    D[b] = x + z[b];
+    if (b < 3) sub = __builtin_amdgcn_mfma_f32_16x16x4f32(LoT[b], D[b], sub, 0, 0, 0);
+  }
+  return D;
 }
 
 // Loads whose width does not depend on a runtime dtype, so every dtype takes one code path and the compiler has no
@@ -180,6 +206,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   using PT = PoolTerms<Tpool>;
   __shared__ float4 s_nd[NP];    // per node: ks, qs, beta, log G
   __shared__ uint32_t s_anc[NP];  // per node: strict ancestors
+  __shared__ int s_id[NP];        // position -> row of the request
 
   // Work item: consecutive items share a key head (value heads of one group, then column slices); the hardware deals
   // workgroups to the 8 XCDs in turn, so item = (block % 8) * per_xcd + block / 8 gives each XCD one contiguous run.
@@ -202,13 +229,19 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   if (T <= 0) return;
 
   // ---- every other load before the first wait -------------------------------------------------------------------
-  const int ct = c < T ? c : T - 1;  // lanes past the tree read its last node (finite values, masked below)
-  const int64_t tok = bos + ct;
-  const int par_raw = entry(a.parent, n, ct);
-  const Word ga = word_of(a.a, tok * a.stride_a + hv, a.gate_dtype);
-  const Word gb = word_of(a.b, tok * a.stride_b + hv, a.gate_dtype);
+  const int par_raw = entry(a.parent, n, c < T ? c : T - 1);  // lane c is row c here
+  Word ga, gb;
   uint4 qr[KB], kr[KB];
-  {
+  Run16<NTL> vr[4];
+  const int v0 = slice * 16 * NTL;
+  auto load_rows = [&](auto&& row_of) {  // row_of(position): the request's row there, or one past the tree, where the
+    auto row_at = [&](int p) {           // last row is read (finite values, masked below)
+      const int row = row_of(p);
+      return bos + (row < T ? row : T - 1);
+    };
+    const int64_t tok = row_at(c);
+    ga = word_of(a.a, tok * a.stride_a + hv, a.gate_dtype);
+    gb = word_of(a.b, tok * a.stride_b + hv, a.gate_dtype);
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + tok * a.stride_q + ih * K + 8 * g;
     const uint16_t* kp = static_cast<const uint16_t*>(a.k) + tok * a.stride_k + ih * K + 8 * g;
 #pragma unroll
@@ -216,16 +249,13 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
       qr[kb] = *reinterpret_cast<const uint4*>(qp + 32 * kb);
       kr[kb] = *reinterpret_cast<const uint4*>(kp + 32 * kb);
     }
-  }
-  // v before the pool slice: loads complete in order, and the first tile needs v but only its own slice part
-  const int v0 = slice * 16 * NTL;
-  Run16<NTL> vr[4];
+    // v before the pool slice: loads complete in order, and the first tile needs v but only its own slice part
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = 4 * g + r;
-    const int64_t ti = bos + (i < T ? i : T - 1);
-    vr[r].load(static_cast<const uint16_t*>(a.v) + ti * a.stride_v + static_cast<int64_t>(hv) * a.V + v0 + NTL * c);
-  }
+    for (int r = 0; r < 4; ++r)
+      vr[r].load(static_cast<const uint16_t*>(a.v) + row_at(4 * g + r) * a.stride_v + static_cast<int64_t>(hv) * a.V + v0 +
+                 NTL * c);
+  };
+  load_rows(place);
   // The pool slice (rows v0 .. v0 + 16 NTL of the request's slot) through a buffer resource whose range is the slice,
   // or empty for a negative slot index: its loads then return zeros, the zero initial state (:341-345), with no
   // branch around them.
@@ -249,6 +279,34 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   // keep the scheduler from sinking these loads below the per-node math that waits for the q / k rows
   __builtin_amdgcn_sched_barrier(0);
 
+  // ---- the order of the nodes: parents first -------------------------------------------------------------------------
+  // a parent outside the tree (or the node itself) makes the node a root
+  const int par_row = c > 0 && c < T && par_raw >= 0 && par_raw < T && par_raw != c ? par_raw : -1;
+  int row_c = place(c), par;  // from here on lane c is the node at position c: its row, its parent's position
+  if (__ballot(par_row > c) == 0) {
+    const int up = __shfl(par_row, row_c, 16);
+    par = up >= 0 ? place(up) : -1;
+  } else {  // rank the rows by (depth, row)
+    int depth = 0;
+    for (int it = 0, x = par_row; it < T; ++it) {  // one step up for every lane; all lanes take part in the shuffle
+      const int up = __shfl(par_row, x >= 0 ? x : 0, 16);
+      if (x >= 0) {
+        ++depth;
+        x = up;
+      }
+    }
+    const int key = c < T ? depth * 16 + c : 16 * 32 + c;
+    int rank = 0;
+    for (int j = 0; j < 16; ++j) rank += readlane(key, j) < key ? 1 : 0;
+    s_id[place(rank)] = c;
+    __syncthreads();
+    row_c = s_id[c];
+    const int up = __shfl(par_row, row_c, 16), up_rank = __shfl(rank, up >= 0 ? up : 0, 16);
+    par = up >= 0 ? place(up_rank) : -1;
+    load_rows([&](int p) { return s_id[p]; });
+  }
+  const bool in = place(c) < T;  // a rank past the tree's is none of its rows
+
   // ---- node x node products; their diagonals are the squared norms ---------------------------------------------------
   f32x4_t KK = {0.f, 0.f, 0.f, 0.f}, KQ = {0.f, 0.f, 0.f, 0.f}, QQ = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -264,9 +322,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   const uint32_t ga_raw = a.gate_dtype == EAGLE4_F32 ? ga.w : (ga.w >> ga.sh) & 0xffffu;
   const uint32_t gb_raw = a.gate_dtype == EAGLE4_F32 ? gb.w : (gb.w >> gb.sh) & 0xffffu;
   const float2 gt = gate_of(ga_raw, gb_raw, a.gate_dtype, 1.0f, 20.0f, A, dt_bias);
-  const float decay = c < T ? gt.x : 1.0f, beta = c < T ? gt.y : 0.0f;  // past the tree: exp(g) 1, beta 0 (:316-317)
-  // a parent outside the tree (or the node itself) makes the node a root
-  const int par = c > 0 && c < T && par_raw >= 0 && par_raw < T && par_raw != c ? par_raw : -1;
+  const float decay = in ? gt.x : 1.0f, beta = in ? gt.y : 0.0f;  // past the tree: exp(g) 1, beta 0 (:316-317)
   // pointer jumping: after round j, anc holds the ancestors at distance 1 .. 2^j, lsum the log2 decays of the node and
   // its ancestors at distance < 2^j, jmp the ancestor at distance 2^j (-1 past the root); depth < 16 needs 4 rounds.
   // Decay ratios are then powers of two of log2 differences (the hardware exp2 / log2, ~1 ulp).
@@ -293,13 +349,14 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   if (g == (c >> 2)) {
     s_nd[c] = make_float4(1.0f / sqrtf(kk + 1e-6f), a.scale / sqrtf(qq + 1e-6f), beta, logG);  // (:147-150)
     s_anc[c] = anc;
+    s_id[c] = row_c;
   }
   __syncthreads();
   const float ks = s_nd[c].x, qs = s_nd[c].y;
   // the record's key and decay (once per node and value head) leave now, ahead of the matrix work
   float* rec = a.records + static_cast<int64_t>(rec_row) * a.stride_records_row;
-  if (slice == 0 && rec_row >= 0 && c < T) {
-    float* p = rec + (static_cast<int64_t>(c) * a.HV + hv) * a.rec + a.V;
+  if (slice == 0 && rec_row >= 0 && in) {
+    float* p = rec + (static_cast<int64_t>(row_c) * a.HV + hv) * a.rec + a.V;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const uint4 x = kr[kb];
@@ -313,7 +370,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   // ---- L, L^T, W^T -------------------------------------------------------------------------------------------------
   float4 nd[4];
   float Gr[4];
-  f32x4_t L, LT, WT, I;
+  f32x4_t B, BT, LoT, WT;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = 4 * g + r;
@@ -324,22 +381,19 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
     const bool i_above_c = (anc >> i) & 1u;    // i a strict ancestor of c
     const float kk_n = nd[r].x * ks * KK[r];
     // L[i][c] = beta_i G_i / G_c k^_i . k^_c on strict ancestors c of i
-    L[r] = c_above_i ? nd[r].z * __builtin_amdgcn_exp2f(nd[r].w - logG) * kk_n : 0.f;
+    const float l = c_above_i ? nd[r].z * __builtin_amdgcn_exp2f(nd[r].w - logG) * kk_n : 0.f;
     // L^T[i][c] = L[c][i];  W^T[i][c] = W[c][i] = G_c / G_i q^_c . k^_i on ancestors-or-self i of c
     const float ratio = i_above_c || i == c ? __builtin_amdgcn_exp2f(logG - nd[r].w) : 0.f;
-    LT[r] = i_above_c ? beta * ratio * kk_n : 0.f;
+    const float lt = i_above_c ? beta * ratio * kk_n : 0.f;
+    const bool own = (c & 3) == r;  // nodes i and c in one block of four
+    B[r] = own ? l : 0.f;
+    BT[r] = own ? lt : 0.f;
+    LoT[r] = own ? 0.f : lt;
     WT[r] = ratio * (qs * nd[r].x * KQ[r]);
-    I[r] = i == c ? 1.f : 0.f;
   }
-  // Tinv^T = (I + P8^T)(I + P4^T)(I + P2^T)(I - L^T), P2 = L L, P4 = P2 P2, P8 = P4 P4 (powers of L commute)
-  const f32x4_t P2 = mm(LT, L), P2T = mm(L, LT);
-  const f32x4_t P4 = mm(P2T, P2), P4T = mm(P2, P2T);
-  const f32x4_t P8 = mm(P4T, P4);
-  f32x4_t TinvT = mm(I + P2, I - LT);
-  TinvT = mm(I + P4, TinvT);
-  TinvT = mm(I + P8, TinvT);
+  const f32x4_t invT = block_inverses(B, BT);
 
-  // ---- per 16-column tile: K S0^T, Q S0^T, rhs, D = Tinv rhs, O = G Q S0^T + W D ------------------------------------
+  // ---- per 16-column tile: K S0^T, Q S0^T, rhs, D, O = G Q S0^T + W D ------------------------------------
   float D[4][NTL], O[4][NTL];
 #pragma unroll
   for (int u = 0; u < NTL; ++u) {
@@ -357,8 +411,8 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
     f32x4_t rhs;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      rhs[r] = 4 * g + r < T ? nd[r].z * (vr[r].at(u) - Gr[r] * (nd[r].x * KS[r])) : 0.f;
-    const f32x4_t Dt = mm(TinvT, rhs);
+      rhs[r] = 4 * r + g < T ? nd[r].z * (vr[r].at(u) - Gr[r] * (nd[r].x * KS[r])) : 0.f;
+    const f32x4_t Dt = solve_tile(invT, LoT, rhs, f32x4_t{0.f, 0.f, 0.f, 0.f});
     const f32x4_t Wd = mm(WT, Dt);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -371,8 +425,8 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   const int64_t col = static_cast<int64_t>(hv) * a.V + v0 + NTL * c;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int i = 4 * g + r;
-    if (i < T) {
+    if (4 * r + g < T) {
+      const int i = s_id[4 * g + r];
       store_run_out<NTL>(a.out, (bos + i) * a.stride_o + col, a.out_dtype, O[r]);
       if (rec_row >= 0) store_run_f32<NTL>(rec + (static_cast<int64_t>(i) * a.HV + hv) * a.rec + v0 + NTL * c, D[r]);
     }
@@ -423,21 +477,12 @@ int launch_k(const eagle4_records_args& a, hipStream_t s) {
 // column tiles) and, with few requests, by their dependence; the walk that it replaces steps through the nodes one by
 // one, each a chain of two lane sums. K = V = 128, fp32 pool, one call among others: 1 request of 24 nodes, 16 heads
 // 33.4 -> 9.4 us; 8 of 40 nodes, 48 heads 318 -> 31 us; 32 of 64 nodes, 48 heads 2108 -> 157 us.
-//   - A diagonal tile is solved by substitution over blocks of four nodes, each block by its own inverse
-//     (I + B)^-1 = I - B + B^2 - B^3. The product form of a whole tile's inverse (powers up to L^8) cancels where keys along
-//     a path are alike and gates near one: a chain of 40 nodes, keys 0.9 alike, beta and decay 1, has powers in the
-//     thousands, and deltas of order one were off by 1e-3; by substitution 1.5e-6 (the walk in fp32: 4e-7).
 //   - Decay ratios are exp2 of differences of root-path sums of log2 decays; the sums are fp64, so what two nodes share
 //     cancels exactly and the ratio's error is that of the path between them, whatever the root path's length.
 //   - A value that is not finite stays on its node and the node's descendants, as in a walk: products with zeros would
 //     spread it over the tile, so it is taken out of the right-hand sides (and a node with such a key or gate out of
 //     the products), remembered per column, and put back where the outputs of that path are stored: NaN, as in the walk,
 //     whose states then hold infinities of both signs; the delta of an infinite value itself stays infinite.
-// The node at position p of the wide form's 16-row tiles (and the position of a node: its own inverse): rows 4 g + b of
-// a tile, element b of the lanes, hold nodes 4 b + g, so that what one MFMA contracts over (element b of the four lane
-// groups) is a block of four consecutive nodes.
-E4_DEV int place(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
-
 template <int K, int NTL, int NTILE, typename Tpool>
 __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records_args a, int slices, int per_xcd,
                                                              int total) {
@@ -731,9 +776,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
       LoT[r] = own ? 0.f : lt;
       WT[r] = i_above_c || i == c ? ratio * (ci.y * nd[r].x * KQ[r]) : 0.f;
     }
-    // (I + B)^-1 - I = B^2 - B - B B^2 for the 4 x 4 blocks B on L_II's diagonal (B^4 = 0), transposed
-    const f32x4_t B2T = mm(B, BT);
-    const f32x4_t invT = mm(B, -B2T, B2T - BT);
+    const f32x4_t invT = block_inverses(B, BT);
 #pragma unroll
     for (int u = 0; u < NTL; ++u) {
       f32x4_t rhs;
@@ -757,14 +800,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
         lost[u] |= static_cast<uint64_t>(m) << (16 * I);
         any_lost = true;
       }
-      // element b of the lanes is block b: its right-hand side less what the blocks before it give, then its inverse
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const float x = rhs[b] - sub[u][b];
-        const f32x4_t z = __builtin_amdgcn_mfma_f32_16x16x4f32(invT[b], x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        D[I][u][b] = x + z[b];
-        if (b < 3) sub[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(LoT[b], D[I][u][b], sub[u], 0, 0, 0);
-      }
+      D[I][u] = solve_tile(invT, LoT, rhs, sub[u]);
       out[u] = mm(WT, D[I][u], out[u]);
     }
     // ---- the tile's outputs and deltas ----

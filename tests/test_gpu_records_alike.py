@@ -42,7 +42,9 @@ def _walk64(inp, width, K, V):
 @pytest.mark.parametrize("alike,b,a", [(0.9, 8.0, -8.0), (0.99, 4.0, -4.0), (0.999, 8.0, -12.0), (0.5, 8.0, -8.0)])
 @pytest.mark.parametrize("width,n,dims,pool_dtype", [
     (40, 3, (1, 2, 128, 32), torch.float32), (64, 2, (2, 2, 64, 16), torch.bfloat16), (24, 2, (1, 2, 32, 48), torch.float16),
-    (48, 8, (4, 32, 128, 64), torch.float32)])  # the last: two column tiles a wave
+    (48, 8, (4, 32, 128, 64), torch.float32),  # two column tiles a wave
+    (16, 3, (1, 2, 128, 32), torch.float32), (13, 4, (2, 2, 256, 16), torch.bfloat16),  # one tile of nodes
+    (9, 32, (4, 16, 64, 32), torch.float32), (16, 64, (4, 16, 128, 64), torch.bfloat16)])  # two and four column tiles
 def test_alike_keys_keep_their_deltas(dev, alike, b, a, width, n, dims, pool_dtype):
     from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
 
