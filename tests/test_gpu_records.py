@@ -211,10 +211,10 @@ def _relabelled_tree(rng, n):
     return par
 
 
-def _chunk_case(dev, trees, dims, pool_dtype, seed, edit=None):
+def _chunk_case(dev, trees, dims, pool_dtype, seed, edit=None, in_dtype=torch.bfloat16):
     from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
 
-    inp, width = _inputs(trees, *dims, pool_dtype, seed=seed)
+    inp, width = _inputs(trees, *dims, pool_dtype, in_dtype=in_dtype, seed=seed)
     if edit is not None:
         edit(inp)
     want_rec = inp["records"].clone()
@@ -265,12 +265,29 @@ def test_chunk_form_batch_tilings(dev, pool_dtype):
     _chunk_case(dev, trees, (4, 16, 128, 128), pool_dtype, 52)
 
 
-def test_chunk_form_wide_trees_walk(dev):
-    """Trees wider than 16 nodes take the depth-first walk; the same closed form."""
+def test_chunk_form_wide_trees(dev):
+    """Trees wider than 16 nodes; the same closed form, tile by tile."""
     announce("records chunk form width 24")
     rng = np.random.default_rng(41)
     trees = [seeded_tree(rng, 24), seeded_tree(rng, 20), [-1, 0, 0, 1]]
     _chunk_case(dev, trees, (2, 4, 128, 128), torch.float32, 42)
+
+
+@pytest.mark.parametrize("pool_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dims,in_dtype", [((2, 4, 128, 32), torch.float16), ((1, 2, 64, 24), torch.float32),
+                                           ((1, 2, 256, 16), torch.bfloat16), ((1, 3, 16, 16), torch.bfloat16)])
+def test_chunk_form_by_the_walk(dev, dims, in_dtype, pool_dtype):
+    """What the matrix cores do not cover (inputs that are not bf16, K 256 above 16 nodes, K below 32) walks the nodes,
+    unrounded: width 24, branches nested deeper than the parked states, parents after their children."""
+    announce(f"records chunk form by the walk dims={dims} {in_dtype} pool={pool_dtype}")
+    rng = np.random.default_rng(43)
+    trees = [_nested_branches(7), _relabelled_tree(rng, 24), seeded_tree(rng, 24), [-1], [], _nested_branches(5)]
+
+    def edit(inp):
+        inp["state_indices"][2] = -1
+        inp["record_indices"][5] = -1
+
+    _chunk_case(dev, trees, dims, pool_dtype, 44, edit, in_dtype)
 
 
 def test_deep_branching_replays_unparked_parents(dev):

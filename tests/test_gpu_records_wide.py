@@ -30,34 +30,53 @@ def test_wide_trees_match_the_closed_form(dev, width, dims, pool_dtype):
     _chunk_case(dev, trees, dims, pool_dtype, width, edit)
 
 
+@pytest.mark.parametrize("width", [24, 40, 64])
+@pytest.mark.parametrize("pool_dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_two_column_tiles_a_wave(dev, width, pool_dtype):
+    """16 requests of 16 value heads and V 64: 512 waves of two column tiles, from where on a wave takes two."""
+    announce(f"records chunk form width {width}, two column tiles, pool={pool_dtype}")
+    rng = np.random.default_rng(width)
+    trees = [(_relabelled_tree if i % 3 == 1 else seeded_tree)(rng, int(rng.integers(max(2, width - 20), width + 1)))
+             for i in range(14)] + [list(range(-1, width - 1)), []]
+
+    def edit(inp):
+        inp["state_indices"][3] = -1  # no pool slot: zeros
+        inp["record_indices"][4] = -1  # outputs only
+
+    _chunk_case(dev, trees, (4, 16, 128, 64), pool_dtype, width + 1, edit)
+
+
+@pytest.mark.parametrize("n,H,HV,V", [(1, 1, 2, 32), (16, 2, 16, 64)])  # one and two column tiles a wave
 @pytest.mark.parametrize("what", ["v", "k", "a"])
-def test_values_that_are_not_finite_stay_on_their_path(dev, what):
+def test_values_that_are_not_finite_stay_on_their_path(dev, what, n, H, HV, V):
     """One node's value, key or gate not finite: the node and its descendants get outputs that are not finite in the
     columns concerned, every other output keeps its bits."""
     from eagle_harness.kernels.gdn_tree_records import gdn_tree_chunk_update
 
     announce(f"records chunk form, {what} not finite")
     tree = [-1, 0, 1, 2, 0, 4, 5] + list(range(6, 30)) + [0, 31, 32]  # node 3's chain ends; 4 .. 30 one chain; 31 .. 33
-    inp, width = _inputs([tree], 1, 2, 128, 32, torch.float32, seed=3)
+    inp, width = _inputs([tree] * n, H, HV, 128, V, torch.float32, seed=3)
     clean = _to(inp, dev)
     want = _call(gdn_tree_chunk_update, clean, width)
-    node = 5
-    {"v": inp["v"][0, node, 1], "k": inp["k"][0, node, 0], "a": inp["a"][node]}[what][1] = float("nan")
+    request, node = n // 2, 5
+    at = request * len(tree) + node
+    {"v": inp["v"][0, at, 1], "k": inp["k"][0, at, 0], "a": inp["a"][at]}[what][1] = float("nan")  # column 1, the odd one
     g = _to(inp, dev)
     g["records"].fill_(0.0)
     got = _call(gdn_tree_chunk_update, g, width)
     torch.cuda.synchronize()
-    hit = torch.zeros(len(tree), 2, 32, dtype=torch.bool, device=dev)
+    hit = torch.zeros(n, len(tree), HV, V, dtype=torch.bool, device=dev)
     below = [node]
     for j in range(node + 1, len(tree)):
         if tree[j] in below:
             below.append(j)
-    cols = {"v": (slice(1, 2), slice(1, 2)), "k": (slice(0, 2), slice(0, 32)), "a": (slice(1, 2), slice(0, 32))}[what]
-    hit[below, cols[0], cols[1]] = True
-    assert torch.equal(got[0].isnan(), hit)
-    assert torch.equal(got[0][~hit], want[0][~hit])
-    row = int(inp["record_indices"][0])
-    assert torch.equal(g["records"][row, : len(tree), :, :32].isnan(), hit)
+    cols = {"v": (slice(1, 2), slice(1, 2)), "k": (slice(0, HV // H), slice(0, V)), "a": (slice(1, 2), slice(0, V))}[what]
+    hit[request][below, cols[0], cols[1]] = True
+    flat = hit.view(n * len(tree), HV, V)
+    assert torch.equal(got[0].isnan(), flat)
+    assert torch.equal(got[0][~flat], want[0][~flat])
+    rows = inp["record_indices"].long()
+    assert torch.equal(g["records"][rows, : len(tree), :, :V].isnan(), hit)
 
 
 @pytest.mark.parametrize("dims,n", [((1, 2, 128, 32), 1), ((2, 16, 64, 64), 16)])  # one and two column tiles a wave
