@@ -18,8 +18,9 @@ E4_DEV bool better(float v, int64_t i, float bv, int64_t bi) {
 
 // One workgroup of NT threads per row, HBM-bound from about 1000 rows on (vocabulary 151936, bf16, with the tree walk:
 // 4096 rows 233 -> 189 us, 6.6 TB/s; 256 rows 74 -> 18 us, 16 rows 62 -> 12 us, where four waves a row and the search of
-// nearly every vector had bound it; 50257, 256 rows, most of them not on 16 bytes: 81 -> 11 us). A row that does not start on a 16-byte boundary (an odd vocabulary) has its first
-// elements, up to the boundary, read one by one, as the last ones past the last whole vector are.
+// nearly every vector had bound it; 50257, 256 rows, most of them not on 16 bytes: 81 -> 11 us). A row that does not
+// start on a 16-byte boundary (an odd vocabulary) has its first elements, up to the boundary, read one by one, as the
+// last ones past the last whole vector are.
 template <typename T, int NT>
 __global__ __launch_bounds__(NT) void argmax_kernel(const eagle4_argmax_args a) {
   using S = typename T::storage;

@@ -310,16 +310,16 @@ E4_DEV bool merge_partials(int n, PartOf part_of, const float* part_out, const f
   return true;
 }
 
-// The runs per row for rows of about `partials` each, `rows` rows in all: one where a thread takes them in one round trip,
-// else as many as a workgroup holds (up to 16) or four, as long as that makes fewer than 2048 workgroups (from there on
-// starting them costs more than the round trips: 64 segments of 96 rows over 5 pieces at D 256, 6144 workgroups of four
-// runs 15.6 us, 9.7 without). `go` gets the number as a type tag.
+// The runs per row for rows of about `partials` each, `rows` rows in all: one up to `four` partials (a thread takes
+// kMergeGroup of them in one round trip), four beyond, beyond `most` as many as a workgroup holds (up to 16), as long as
+// that makes fewer than 2048 workgroups (from there on starting them costs more than the round trips: 64 segments of 96
+// rows over 5 pieces at D 256, 6144 workgroups of four runs 15.6 us, 9.7 without). `go` gets the number as a type tag.
 template <int D, typename F>
-int with_merge_runs(int64_t partials, int64_t rows, F&& go) {
+int with_merge_runs(int64_t partials, int64_t rows, F&& go, int64_t four = kMergeGroup, int64_t most = 4 * kMergeGroup) {
   constexpr int kMost = 1024 / D < 16 ? 1024 / D : 16;
   const auto groups = [&](int runs) { return rows * runs * (D / 4) / 256; };
-  if (partials > 4 * kMergeGroup && groups(kMost) < 2048) return go(std::integral_constant<int, kMost>{});
-  if (partials > kMergeGroup && groups(4) < 2048) return go(std::integral_constant<int, 4>{});
+  if (partials > most && groups(kMost) < 2048) return go(std::integral_constant<int, kMost>{});
+  if (partials > four && groups(4) < 2048) return go(std::integral_constant<int, 4>{});
   return go(std::integral_constant<int, 1>{});
 }
 

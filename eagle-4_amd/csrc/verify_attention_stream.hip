@@ -1260,11 +1260,14 @@ int launch(const eagle4_attn_args& a, const StreamPlan& p, hipStream_t s) {
   // of 1024 at D 64, 9 pieces 6.2 -> 4.4 us).
   const int64_t segs = static_cast<int64_t>(a.num_reqs) * p.HR, pieces = p.nwg / segs + 1;
   if (pieces > 2)
-    return with_merge_runs<D>(pieces > 4 ? pieces + kMergeGroup : 1, segs * p.rows_seg, [&](auto runs) {
-      constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
-      verify_stream_merge_many<D, SG, T><<<dim3(segs, e4::ceil_div(p.rows_seg, RPB)), 256, 0, s>>>(a, p);
-      return E4_LAUNCH_STATUS();
-    });
+    return with_merge_runs<D>(
+        pieces, segs * p.rows_seg,
+        [&](auto runs) {
+          constexpr int SG = decltype(runs)::value, RPB = 256 / (D / 4) / SG;
+          verify_stream_merge_many<D, SG, T><<<dim3(segs, e4::ceil_div(p.rows_seg, RPB)), 256, 0, s>>>(a, p);
+          return E4_LAUNCH_STATUS();
+        },
+        4, 24);
   constexpr int kMergeThreadsPerRow = D / (D < 16 ? D : 16);
   verify_stream_merge<D, T><<<dim3(segs, e4::ceil_div(static_cast<int64_t>(p.rows_seg) * kMergeThreadsPerRow, 256)), 256,
                               0, s>>>(a, p);
