@@ -304,13 +304,18 @@ __global__ __launch_bounds__(256) void compact_rows_kernel(const eagle4_compact_
 
 // 16 waves on rows of 200 KB and more, 8 on shorter ones, whose 16 waves would spend more on their own reduction than on
 // the row (bf16, us with the tree walk, 8 / 16 waves: vocabulary 151936, 16 rows 12.3 / 11.7, 256 rows 18.7 / 18.3, 4096
-// rows 193 / 189; 50257, 16 rows 9.1 / 9.3, 4096 rows 69 / 72; 32000, 4096 rows 45 / 55). 4 waves were slower in all.
+// rows 193 / 189; 50257, 16 rows 9.1 / 9.3, 4096 rows 69 / 72; 32000, 4096 rows 45 / 55), 4 where those read a row in one
+// group of loads (the targets alone, 4 / 8 waves: 8192, 16 rows 4.5 / 4.9, 4096 rows 13.4 / 20.9; 512, 4096 rows 8.3 /
+// 13.7; fp32, 4096, 4096 rows 12.2 / 18.1).
 template <typename T>
 int launch_argmax(const eagle4_argmax_args& a, hipStream_t s) {
-  if (static_cast<int64_t>(a.vocab) * static_cast<int64_t>(sizeof(typename T::storage)) >= 200 * 1024)
+  const int64_t bytes = static_cast<int64_t>(a.vocab) * static_cast<int64_t>(sizeof(typename T::storage));
+  if (bytes >= 200 * 1024)
     argmax_kernel<T, 1024><<<a.rows, 1024, 0, s>>>(a);
-  else
+  else if (bytes > 16 * 1024)
     argmax_kernel<T, 512><<<a.rows, 512, 0, s>>>(a);
+  else
+    argmax_kernel<T, 256><<<a.rows, 256, 0, s>>>(a);
   return E4_LAUNCH_STATUS();
 }
 
