@@ -69,16 +69,17 @@ E4_DEV f32x4_t block_inverses(f32x4_t B, f32x4_t BT) {
   const f32x4_t B2T = mm(B, BT);
   return mm(B, -B2T, B2T - BT);
 }
-E4_DEV f32x4_t solve_tile(f32x4_t invT, f32x4_t LoT, f32x4_t rhs, f32x4_t sub) {
-  f32x4_t D;
+template <int N>
+E4_DEV void solve_tiles(f32x4_t invT, f32x4_t LoT, const f32x4_t (&rhs)[N], f32x4_t (&sub)[N], f32x4_t (&D)[N]) {
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const float x = rhs[b] - sub[b];
-    const f32x4_t z = __builtin_amdgcn_mfma_f32_16x16x4f32(invT[b], x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    D[b] = x + z[b];
-    if (b < 3) sub = __builtin_amdgcn_mfma_f32_16x16x4f32(LoT[b], D[b], sub, 0, 0, 0);
-  }
-  return D;
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int u = 0; u < N; ++u) {  // column tiles: independent chains
+      const float x = rhs[u][b] - sub[u][b];
+      const f32x4_t z = __builtin_amdgcn_mfma_f32_16x16x4f32(invT[b], x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      D[u][b] = x + z[b];
+      if (b < 3) sub[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(LoT[b], D[u][b], sub[u], 0, 0, 0);
+    }
 }
 
 // Loads whose width does not depend on a runtime dtype, so every dtype takes one code path and the compiler has no
@@ -304,6 +305,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
     const int up = __shfl(par_row, row_c, 16), up_rank = __shfl(rank, up >= 0 ? up : 0, 16);
     par = up >= 0 ? place(up_rank) : -1;
     load_rows([&](int p) { return s_id[p]; });
+    settle_loads();  // else the waits after the join would take the common path's first loads for its last
   }
   const bool in = place(c) < T;  // a rank past the tree's is none of its rows
 
@@ -394,7 +396,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   const f32x4_t invT = block_inverses(B, BT);
 
   // ---- per 16-column tile: K S0^T, Q S0^T, rhs, D, O = G Q S0^T + W D ------------------------------------
-  float D[4][NTL], O[4][NTL];
+  f32x4_t rhs[NTL], D[NTL], O[NTL], sub[NTL];
 #pragma unroll
   for (int u = 0; u < NTL; ++u) {
     f32x4_t KS = {0.f, 0.f, 0.f, 0.f}, QS = {0.f, 0.f, 0.f, 0.f};
@@ -408,18 +410,16 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
         QS = mma_bf16(qr[kb], st[s], QS);
       }
     }
-    f32x4_t rhs;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      rhs[r] = 4 * r + g < T ? nd[r].z * (vr[r].at(u) - Gr[r] * (nd[r].x * KS[r])) : 0.f;
-    const f32x4_t Dt = solve_tile(invT, LoT, rhs, f32x4_t{0.f, 0.f, 0.f, 0.f});
-    const f32x4_t Wd = mm(WT, Dt);
+    sub[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      D[r][u] = Dt[r];
-      O[r][u] = Gr[r] * (nd[r].y * QS[r]) + Wd[r];
+      rhs[u][r] = 4 * r + g < T ? nd[r].z * (vr[r].at(u) - Gr[r] * (nd[r].x * KS[r])) : 0.f;
+      O[u][r] = Gr[r] * (nd[r].y * QS[r]);
     }
   }
+  solve_tiles<NTL>(invT, LoT, rhs, sub, D);
+#pragma unroll
+  for (int u = 0; u < NTL; ++u) O[u] += mm(WT, D[u]);
 
   // ---- stores --------------------------------------------------------------------------------------------------------
   const int64_t col = static_cast<int64_t>(hv) * a.V + v0 + NTL * c;
@@ -427,8 +427,14 @@ __global__ __launch_bounds__(64) void gdn_chunk_kernel(const eagle4_records_args
   for (int r = 0; r < 4; ++r) {
     if (4 * r + g < T) {
       const int i = s_id[4 * g + r];
-      store_run_out<NTL>(a.out, (bos + i) * a.stride_o + col, a.out_dtype, O[r]);
-      if (rec_row >= 0) store_run_f32<NTL>(rec + (static_cast<int64_t>(i) * a.HV + hv) * a.rec + v0 + NTL * c, D[r]);
+      float o[NTL], d[NTL];
+#pragma unroll
+      for (int u = 0; u < NTL; ++u) {
+        o[u] = O[u][r];
+        d[u] = D[u][r];
+      }
+      store_run_out<NTL>(a.out, (bos + i) * a.stride_o + col, a.out_dtype, o);
+      if (rec_row >= 0) store_run_f32<NTL>(rec + (static_cast<int64_t>(i) * a.HV + hv) * a.rec + v0 + NTL * c, d);
     }
   }
 }
@@ -726,7 +732,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
     const float4 ci = s_nd[16 * I + c];  // the node of this lane's column
     const double lg_c = s_lg[16 * I + c];
     const uint64_t anc_c = s_anc[16 * I + c];
-    f32x4_t sub[NTL], out[NTL];
+    f32x4_t sub[NTL], out[NTL], rhs[NTL];
 #pragma unroll
     for (int u = 0; u < NTL; ++u) {
       sub[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -781,30 +787,30 @@ __global__ __launch_bounds__(64) void gdn_chunk_wide_kernel(const eagle4_records
     const f32x4_t invT = block_inverses(B, BT);
 #pragma unroll
     for (int u = 0; u < NTL; ++u) {
-      f32x4_t rhs;
       bool off = false;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        rhs[r] = 16 * I + 4 * r + g < T ? nd[r].z * (vr[I][r].at(u) - nd[r].w * (nd[r].x * KS[I][u][r])) : 0.f;
-        off |= !(fabsf(rhs[r] - sub[u][r]) <= 3.4e38f);
+        rhs[u][r] = 16 * I + 4 * r + g < T ? nd[r].z * (vr[I][r].at(u) - nd[r].w * (nd[r].x * KS[I][u][r])) : 0.f;
+        off |= !(fabsf(rhs[u][r] - sub[u][r]) <= 3.4e38f);
       }
       if (__ballot(off) != 0) {  // take what is not finite out of the products, remember where it was
         uint32_t m = 0;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (!(fabsf(rhs[r] - sub[u][r]) <= 3.4e38f)) {
+          if (!(fabsf(rhs[u][r] - sub[u][r]) <= 3.4e38f)) {
             m |= 1u << (4 * g + r);
-            s_raw[u][r][lane] = rhs[r] - sub[u][r];
-            rhs[r] = sub[u][r] = 0.f;
+            s_raw[u][r][lane] = rhs[u][r] - sub[u][r];
+            rhs[u][r] = sub[u][r] = 0.f;
           }
         m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 16));
         m |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32));
         lost[u] |= static_cast<uint64_t>(m) << (16 * I);
         any_lost = true;
       }
-      D[I][u] = solve_tile(invT, LoT, rhs, sub[u]);
-      out[u] = mm(WT, D[I][u], out[u]);
     }
+    solve_tiles<NTL>(invT, LoT, rhs, sub, D[I]);
+#pragma unroll
+    for (int u = 0; u < NTL; ++u) out[u] = mm(WT, D[I][u], out[u]);
     // ---- the tile's outputs and deltas ----
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
