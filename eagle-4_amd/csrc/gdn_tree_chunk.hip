@@ -481,10 +481,10 @@ int launch_k(const eagle4_records_args& a, hipStream_t s) {
 // wave's NTL column tiles, nothing is kept but D). One wave per (request, value head, 16 NTL columns). Rows given in
 // another order are first ranked by depth. Bound by one wave's latency: at K 128 and three or four tiles a wave holds 250
 // to 300 registers, so one or two fit a SIMD, and the tiles are a serial chain. Of a wave's cycles at 8 requests of 20 - 40
-// nodes, 32 heads (at 32 of 64 nodes, 48 heads) the MFMA is busy for 19 % (25), the VALU issues for 25 % (28), and 37 %
-// (28) are waits for loads and LDS. The walk that it replaces steps through the nodes one by one, each a chain of two
+// nodes, 32 heads (at 32 of 64 nodes, 48 heads) the MFMA is busy for 19 % (26), the VALU issues for 25 % (29), and 34 %
+// (26) are waits for loads and LDS. The walk that it replaces steps through the nodes one by one, each a chain of two
 // lane sums. K = V = 128, fp32 pool, kernel against the walk: 1 request of 24 nodes, 16 heads 33.4 -> 8.6 us; 8 of 40
-// nodes, 48 heads 318 -> 29 us; 32 of 64 nodes, 48 heads 2108 -> 144 us.
+// nodes, 48 heads 318 -> 29 us; 32 of 64 nodes, 48 heads 2108 -> 141 us.
 //   - Decay ratios are exp2 of differences of root-path sums of log2 decays; the sums are fp64, so what two nodes share
 //     cancels exactly and the ratio's error is that of the path between them, whatever the root path's length.
 //   - A value that is not finite stays on its node and the node's descendants, as in a walk: products with zeros would

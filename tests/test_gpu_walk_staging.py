@@ -1,5 +1,6 @@
-"""The snapshot walk with 32 staged nodes against 16 (the per-row slot table's columns choose): trees around both counts, in
-both lane forms and pool dtypes, against the same trees under the other count and against the oracle."""
+"""The snapshot walk with 32 staged nodes against 16 (the requests' mean rows choose, at most the per-row slot table's
+columns): trees around both counts, in both lane forms and pool dtypes, bit for bit the same under either count, and
+against the oracle."""
 
 import numpy as np
 import pytest
